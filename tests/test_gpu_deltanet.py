@@ -83,3 +83,94 @@ def test_gated_delta_net_chaining_and_snapshots(gpu, oracle):
     np.testing.assert_array_equal(host(st_all), states[-1])
     for s in range(1, T):
         np.testing.assert_array_equal(host(snap)[s - 1], states[T - 1 - s])
+
+
+def _rule64(q, k, v, g, beta, s0):
+    """The recurrence in float64: q, k [T, n_k, d]; v [T, n_v, d]; returns out, the states after each token."""
+    T, nk, d = q.shape
+    nv = v.shape[1]
+    st, out, states = s0.astype(np.float64), np.zeros((T, nv, d)), []
+    q, k = (np.repeat(x.astype(np.float64), nv // nk, axis=1) for x in (q, k))
+    for t in range(T):
+        st = st * np.exp(g[t].astype(np.float64))[:, None, None]
+        dl = (v[t].astype(np.float64) - np.einsum("hrc,hr->hc", st, k[t])) * beta[t].astype(np.float64)[:, None]
+        st = st + k[t][:, :, None] * dl[:, None, :]
+        out[t] = np.einsum("hrc,hr->hc", st, q[t]) / np.sqrt(d)
+        states.append(st)
+    return out, states
+
+
+def _small(seed, T, nk, nv):
+    rng = np.random.default_rng(seed)
+    qk = rng.standard_normal((2, T, nk, D))
+    qk = (qk / np.linalg.norm(qk, axis=-1, keepdims=True)).astype(np.float32)
+    v = rng.standard_normal((T, nv, D)).astype(np.float32)
+    # a head of long memory, one of short
+    g = (-rng.uniform(0.0, 1.0, (T, nv)) * np.geomspace(0.01, 1.5, nv)).astype(np.float32)
+    beta = rng.uniform(0.0, 1.0, (T, nv)).astype(np.float32)
+    s0 = (rng.standard_normal((nv, D, D)) * 0.05).astype(np.float32)
+    return qk[0], qk[1], v, g, beta, s0
+
+
+def _call(K, q, k, v, g, beta, s0, n_snap=0, pad=0):
+    """pad: extra floats per token in the q, k and v rows (strided views)."""
+    T, nk, _ = q.shape
+    nv = v.shape[1]
+    rows = [np.concatenate([x.reshape(T, -1), np.full((T, pad), np.nan, np.float32)], axis=1) for x in (q, k, v)]
+    qd, kd, vd = (dev(x)[:, :x.shape[1] - pad] for x in rows)
+    st = dev(s0)
+    out = torch.full((T, nv, D), 7.0, dtype=torch.float32, device="cuda")
+    snap = torch.zeros((max(n_snap, 1), nv, D, D), dtype=torch.float32, device="cuda")
+    K.gated_delta_net(qd, kd, vd, dev(g), dev(beta), st, out, nk, snap if n_snap else None, n_snap)
+    return host(out), host(st), host(snap)
+
+
+# chunks of 16 tokens in groups of 64 from 12 tokens on: partial chunks and groups, one and several groups, grids that are and are
+# not a multiple of the 8 XCDs (4 blocks a value head), a last chunk of one token, snapshots behind the chunks
+@pytest.mark.parametrize("T,nk,nv,n_snap,pad", [(11, 1, 2, 0, 0), (12, 1, 3, 0, 4), (15, 2, 2, 0, 0), (16, 1, 2, 0, 8), (17, 1, 1, 0, 0),
+                                                (63, 1, 3, 0, 4), (64, 2, 4, 0, 0), (65, 1, 2, 0, 0), (129, 1, 3, 0, 12),
+                                                (200, 2, 6, 0, 0), (16, 1, 3, 3, 0), (70, 1, 2, 5, 4)])
+def test_gated_delta_net_chunks(gpu, T, nk, nv, n_snap, pad):
+    """Against float64: a token's sums have 128 terms and a state remembers at most T tokens, so the 2-norm error
+    stays within 4 sqrt(128 + T) 2^-24 of the result (5e-6 at T 200; 5e-7 seen at T 512)."""
+    q, k, v, g, beta, s0 = _small(T, T, nk, nv)
+    say(f"gated_delta_net chunks T={T} heads {nk}/{nv} snapshots {n_snap}")
+    out, st, snap = _call(gpu, q, k, v, g, beta, s0, n_snap, pad)
+    r_out, states = _rule64(q, k, v, g, beta, s0)
+    tol = 4 * np.sqrt(128 + T) * 2.0 ** -24
+    for name, a, b in [("out", out, r_out), ("state", st, states[-1])] + \
+            [(f"snap {s}", snap[s - 1], states[T - 1 - s]) for s in range(1, n_snap + 1)]:
+        err = np.linalg.norm(a - b) / np.linalg.norm(b)
+        print(f"  {name} {err:.2e}", flush=True)
+        assert err <= tol, name
+
+
+def test_gated_delta_net_chunks_not_finite(gpu):
+    """A decay of 0 forgets the state exactly; a value that is not finite reaches its own column from its token
+    on, a key every column of its heads, a query its own outputs, and nothing before them."""
+    T, nk, nv = 80, 2, 4
+    q, k, v, g, beta, s0 = _small(3, T, nk, nv)
+    g[37, 1] = -np.inf
+    say("gated_delta_net chunks with a decay of 0")
+    out, st, _ = _call(gpu, q, k, v, g, beta, s0)
+    r_out, states = _rule64(q, k, v, g, beta, s0)
+    tol = 4 * np.sqrt(128 + T) * 2.0 ** -24
+    assert np.linalg.norm(out - r_out) <= tol * np.linalg.norm(r_out)
+    assert np.linalg.norm(st - states[-1]) <= tol * np.linalg.norm(states[-1])
+    v2, k2, q2 = v.copy(), k.copy(), q.copy()
+    v2[21, 0, 5] = np.inf                    # value head 0, column 5
+    k2[42, 1, 9] = np.nan                    # key head 1: value heads 2 and 3
+    q2[10, 0, 3] = np.inf                    # key head 0, token 10 only: value heads 0 and 1
+    say("gated_delta_net chunks with values that are not finite")
+    out2, st2, _ = _call(gpu, q2, k2, v2, g, beta, s0)
+    bad = np.zeros(out.shape, bool)
+    bad[21:, 0, 5] = True
+    bad[42:, 2:] = True
+    bad[10, :2] = True
+    assert not np.isfinite(out2[bad]).any()
+    np.testing.assert_array_equal(out2[~bad], out[~bad])
+    badst = np.zeros(st.shape, bool)
+    badst[0, :, 5] = True
+    badst[2:] = True
+    assert not np.isfinite(st2[badst]).any()
+    np.testing.assert_array_equal(st2[~badst], st[~badst])
