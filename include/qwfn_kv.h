@@ -159,9 +159,12 @@ int qwfn_kv_gather_segments_kv(const void * src_k, const void * src_v, size_t sr
  * a graph, and every ws == NULL call on a device shares that one buffer, so
  * such calls must not overlap (serialise them on one stream). The workspace
  * holds the split partials when the keys are split across workgroups (at
- * least 256 bytes are asked for otherwise); its contents need not be
- * preserved between calls. Calls that run at the same time need distinct
- * workspaces. */
+ * least 256 bytes are asked for otherwise) and, for long query blocks over
+ * many keys, the K/V rows converted once for all of them (800 bytes a key and
+ * KV head, behind the partials: with a workspace that holds only the partials
+ * the call converts them in every workgroup, slower, to the same bits); its
+ * contents need not be preserved between calls. Calls that run at the same
+ * time need distinct workspaces. */
 size_t qwfn_fattn_workspace_size(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,
                                  const qwfn_tensor * mask);
 int qwfn_flash_attn_ext_q8_0(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,

@@ -146,6 +146,8 @@ struct fa_args {
     // a (batch, KV head, row group) on one XCD (they share its query rows)
     int32_t  pre_rgmap;
     uint32_t nbh_mul;      // ceil(2^32 / (B * nh_kv))
+    uint8_t * img;         // k_fa_pre's chunk images [KV head][chunk][IMG_BYTES], or null
+    int32_t  img_chunks;   // chunks of n_kv keys
     // fused append (app_n > 0): F32 rows [nh_kv * D] of K and V quantised into
     // cache rows app_row0 .. app_row0 + app_n - 1 before they are attended
     const char * app_k;
@@ -4056,6 +4058,19 @@ __global__ __launch_bounds__(VS_WAVES * 64, 2) void k_fa_vs(fa_args a) {
 // next key tile (QK) and V block (PV) are issued ahead of the current one's
 // arithmetic. A wave whose rows see none of the
 // chunk's keys (a causal mask's upper triangle) skips it.
+//
+// Where many row groups walk the same chunks (pre_images), the conversion is
+// done once: k_fa_pre_image writes every chunk as k_fa_pre reads it from LDS
+// into the call's workspace, and the key loop is DMAs, one barrier a chunk and
+// the arithmetic. The conversion and its barrier were 1.4 us of a chunk's 6.1;
+// with images a chunk takes 5.0 (64 row groups x 264 chunks, with the image
+// launch and the merge: 380 -> 328 us). Then the SIMDs issue 82% of the time
+// (VALU 67%), the matrix cores are 26% and LDS 44% busy. Measured from there and
+// dropped: the K quants as f16, so that an f16 MFMA gives the exact block dot
+// as a float (128 conversions a wave and chunk fewer, the same bits: 348 against
+// 340 us, for its longer MFMAs and twice the K bytes); the wave priority fixed,
+// off, or high for the younger waves (363 against 354); PV operands read two or
+// three steps ahead, the first ones under the softmax (352, 355 against 349).
 
 constexpr int PRE_WAVES = 8;
 constexpr int PRE_ROWS  = 16 * PRE_WAVES;                 // 128 query rows per block
@@ -4089,6 +4104,29 @@ static_assert(PRE_KB % 1024 == 0, "a tensor's rows of a chunk are whole wave DMA
 static_assert(PRE_WAVES * PRE_QW <= PRE_VT + PRE_KQ, "the query images fit V^T and the K quants");
 static_assert(PRE_CK == 64 && NBLK == PRE_WAVES, "the conversion pass: wave w takes V block w of every key");
 
+// A chunk's image, the converted rows as k_fa_pre reads them from LDS, made
+// once per call by k_fa_pre_image when many row groups share the chunk:
+//   V^T: row d (256) of 64 keys f16 in V^T position order, its 16-byte granule
+//        c at granule c ^ (2 (d & 3));
+//   K quants: [block][key][32], the 8-byte piece j of key k at piece
+//        j ^ ((k >> 2) & 3);
+//   scales: fp16 [K|V][block][key].
+// The two exclusive-ors take the place of the padded row strides above: an
+// operand read serves 128 bytes a clock, 8 lanes of a 16-byte read (4 rows at
+// one granule and 4 at its neighbour) or 16 of an 8-byte read (16 keys), which
+// then fall on 8 granules or 16 pieces of their own; and the image moves to
+// LDS in whole 1 KB DMAs.
+constexpr int IMG_VS    = 2 * PRE_CK;                     // 128: bytes per dim row of V^T
+constexpr int IMG_K     = D * IMG_VS;                     // 32768: K quants' offset
+constexpr int IMG_KS    = QK;                             // 32: bytes per key row of the K quants
+constexpr int IMG_S     = IMG_K + NBLK * PRE_CK * IMG_KS; // 49152: scales' offset
+constexpr int IMG_BYTES = IMG_S + PRE_SKV;                // 51200
+constexpr int IMG_DMA   = IMG_BYTES / 1024;               // 50 wave DMAs
+constexpr int IMG_STAGE = IMG_BYTES + PRE_MDMA * 1024;    // 56320: an image and its mask granules
+constexpr int IMG_SPW   = (IMG_DMA + PRE_MDMA + PRE_WAVES - 1) / PRE_WAVES;   // 7 DMA slots per wave
+static_assert(IMG_BYTES % 1024 == 0, "an image is whole wave DMAs");
+static_assert(PRE_WAVES * PRE_QW <= IMG_STAGE, "the query images fit a stage");
+
 // V^T rows hold a chunk's keys in this order: key k = 32h + 16tt + 4g + i
 // (half h, key tile tt of the half, lane group g, i = 0..3) sits at position
 // 32h + 8g + 4tt + i, so the 8 keys a lane group's PV operand needs are
@@ -4117,16 +4155,118 @@ __device__ __forceinline__ uint32_t cvt_i8_pair(uint32_t s0, uint32_t s1) {
     return d;
 }
 
-template <bool MASKED>
+// The conversion pass of a chunk whose K and V rows (272 bytes each) are in LDS
+// at st: wave w takes V block w (dims 32w .. 32w+31) of the 64 keys: lane (key
+// pair kp, half dh) converts dims 32w + 16dh .. +15 of the keys at V^T
+// positions 2kp, 2kp + 1, and K block w of key `lane` into the repacked
+// quants; lane k also tabulates the K and V scales of block w of key k. Block
+// w's quants start 2 bytes into a word when w is even and on a word boundary
+// when w is odd (34w + 2 = 0 mod 4): the lanes read whole words from the word
+// at or before them and realign them with alignbyte (shift 2 or 0), with no
+// branch on the parity. Rows sit 272 bytes (68 words, 4 banks mod 32) apart,
+// so reads of one offset in many rows would meet in 8 banks: each lane reads
+// its run of words starting at a rotated word (slot i holds word (i + rot) mod
+// n, the word past the run sits in slot n), so that one read's lanes cover
+// every bank. Every read is issued before the first conversion. IMG: the
+// chunk's image at vt (over the rows: a barrier between the reads and the
+// writes), else V^T, K quants and scales with the padded strides.
+template <bool IMG>
+__device__ __forceinline__ void pre_convert(const uint8_t * st, uint8_t * vt, uint8_t * kq,
+                                            uint16_t (* skv)[NBLK][PRE_CK], int lane, int wave) {
+    const int kp = lane & 31, dh = lane >> 5;
+    const int p0 = 2 * kp;
+    // the key at position p0 (its neighbour p0 + 1 is the next key)
+    const int key0 = 32 * (p0 >> 5) + 16 * ((p0 >> 2) & 1) + 4 * ((p0 >> 3) & 3) + (p0 & 3);
+    const int odd = wave & 1;
+    const uint32_t sh = odd ? 0u : 2u;
+    const uint8_t * v0 = st + PRE_KB + key0 * SEG + QBLOCK * wave + 16 * dh + 2 * odd;
+    const uint8_t * k0 = st + lane * SEG + QBLOCK * wave + 2 * odd;
+    const int vrot = (kp >> 3) & 3, krot = (lane >> 3) & 7;
+    uint32_t x[5], y[5], kw[9];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int t = (i + vrot) & 3;
+        x[i] = *(const uint32_t *) (v0 + 4 * t);
+        y[i] = *(const uint32_t *) (v0 + SEG + 4 * t);
+    }
+    x[4] = *(const uint32_t *) (v0 + 16);
+    y[4] = *(const uint32_t *) (v0 + SEG + 16);
+#pragma unroll
+    for (int i = 0; i < 8; i++) kw[i] = *(const uint32_t *) (k0 + 4 * ((i + krot) & 7));
+    kw[8] = *(const uint32_t *) (k0 + 32);
+    const uint16_t dk16 = *(const uint16_t *) (st + lane * SEG + QBLOCK * wave);
+    const uint16_t dv16 = *(const uint16_t *) (st + PRE_KB + lane * SEG + QBLOCK * wave);
+    if constexpr (IMG) __syncthreads();
+    // V: word t of the lane's 16 bytes holds dims 16dh + 4t .. + 3 of keys key0 / key0 + 1
+    constexpr int VS = IMG ? IMG_VS : PRE_VTS;
+    uint8_t * vrow = vt + (32 * wave + 16 * dh) * VS + (IMG ? (2 * p0) & 15 : 2 * p0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int t = (i + vrot) & 3;
+        const uint32_t xa = __builtin_amdgcn_alignbyte(t == 3 ? x[4] : x[(i + 1) & 3], x[i], sh);
+        const uint32_t ya = __builtin_amdgcn_alignbyte(t == 3 ? y[4] : y[(i + 1) & 3], y[i], sh);
+        uint8_t * d = vrow + 4 * t * VS;
+        if constexpr (IMG) {
+            const int c = p0 >> 3;
+            *(uint32_t *) (d + 16 * c) = cvt_i8_pair<0>(xa, ya);
+            *(uint32_t *) (d + VS + 16 * (c ^ 2)) = cvt_i8_pair<1>(xa, ya);
+            *(uint32_t *) (d + 2 * VS + 16 * (c ^ 4)) = cvt_i8_pair<2>(xa, ya);
+            *(uint32_t *) (d + 3 * VS + 16 * (c ^ 6)) = cvt_i8_pair<3>(xa, ya);
+        } else {
+            *(uint32_t *) (d) = cvt_i8_pair<0>(xa, ya);
+            *(uint32_t *) (d + VS) = cvt_i8_pair<1>(xa, ya);
+            *(uint32_t *) (d + 2 * VS) = cvt_i8_pair<2>(xa, ya);
+            *(uint32_t *) (d + 3 * VS) = cvt_i8_pair<3>(xa, ya);
+        }
+    }
+    // K: word t of block w of key `lane` (quants 4t .. 4t + 3) to kq[w][lane]
+    uint8_t * kd = kq + (wave * PRE_CK + lane) * (IMG ? IMG_KS : PRE_KQS);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int t = (i + krot) & 7;
+        const uint32_t q4 = __builtin_amdgcn_alignbyte(t == 7 ? kw[8] : kw[(i + 1) & 7], kw[i], sh);
+        *(uint32_t *) (kd + 4 * (IMG ? t ^ (2 * ((lane >> 2) & 3)) : t)) = q4;   // word t's 8-byte piece is t >> 1
+    }
+    skv[0][wave][lane] = dk16;
+    skv[1][wave][lane] = dv16;
+}
+
+// The images of chunk blockIdx.x of KV head blockIdx.y: the rows to LDS, the
+// conversion over them, the image out. Keys past n_kv are zeros (k_fa_pre masks
+// them). Bound by its bytes (272 + 272 in, 800 out a key and head): 18 us of a
+// profiled launch at 16896 keys and 2 heads, 45 MB.
+__global__ __launch_bounds__(PRE_WAVES * 64) void k_fa_pre_image(fa_args a) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[IMG_BYTES];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c0 = (int64_t) blockIdx.x * PRE_CK;
+    const char * kb = a.k + (size_t) blockIdx.y * a.k_nb2, * vb = a.v + (size_t) blockIdx.y * a.v_nb2;
+    for (int u = threadIdx.x; u < 2 * PRE_KB / 16; u += PRE_WAVES * 64) {
+        const int tensor = u >= PRE_KB / 16;
+        const uint32_t p = (uint32_t) (u - tensor * (PRE_KB / 16)), key = p / 17u, part = p - key * 17u;
+        uint4 x = make_uint4(0, 0, 0, 0);
+        if (c0 + key < a.n_kv)
+            x = *(const uint4 *) ((tensor ? vb + (size_t) (c0 + key) * a.v_nb1 : kb + (size_t) (c0 + key) * a.k_nb1) + 16 * part);
+        *(uint4 *) (lds + 16 * u) = x;
+    }
+    __syncthreads();
+    pre_convert<true>(lds, lds, lds + IMG_K, (uint16_t (*)[NBLK][PRE_CK]) (lds + IMG_S), lane, wave);
+    __syncthreads();
+    uint8_t * out = a.img + ((size_t) blockIdx.y * a.img_chunks + blockIdx.x) * IMG_BYTES;
+    for (int u = threadIdx.x; u < IMG_BYTES / 16; u += PRE_WAVES * 64) *(uint4 *) (out + 16 * u) = *(const uint4 *) (lds + 16 * u);
+}
+
+// IMG: the chunks come as images (one barrier a chunk and no conversion here)
+template <bool MASKED, bool IMG = false>
 __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
     asm volatile("" :: "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.mask), "s"(a.part_o));
-    // V^T | K quants | scales | stage 0 | stage 1; the query images of the
-    // prologue use V^T and the K quants
-    __shared__ __attribute__((aligned(16))) uint8_t lds[PRE_LDS];
-    uint8_t * const vt = lds;
-    uint8_t * const kq = vt + PRE_VT;
-    uint16_t (* const skv)[NBLK][PRE_CK] = (uint16_t (*)[NBLK][PRE_CK]) (kq + PRE_KQ);   // [K|V][block][key] fp16 scales
-    uint8_t * const stg = kq + PRE_KQ + PRE_SKV;
+    // V^T | K quants | scales | stage 0 | stage 1, the query images of the
+    // prologue in V^T and the K quants; or stage 0 | stage 1, each an image
+    // and its mask granules, the query images in stage 1
+    __shared__ __attribute__((aligned(16))) uint8_t lds[IMG ? 2 * IMG_STAGE : PRE_LDS];
+    constexpr int STAGE = IMG ? IMG_STAGE : PRE_STAGE, MOFF = IMG ? IMG_BYTES : PRE_MOFF;
+    constexpr int SPW = IMG ? IMG_SPW : PRE_SPW;
+    constexpr int KQS = IMG ? IMG_KS : PRE_KQS;
+    uint8_t * const stg = IMG ? lds : lds + PRE_VT + PRE_KQ + PRE_SKV;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -4183,20 +4323,25 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
     //      key p / 17), [17, 34) the V rows, then the mask granules (granule
     //      G = 64 m + lane is granule G % 9 of row G / 9; lanes past the rows
     //      re-read the last one). Wave w issues slots w, w + 8, ... ----
-    uint32_t doff[PRE_SPW];
-    bool dlive[PRE_SPW];
+    //      (an image's slots are its 1 KB pieces) ----
+    constexpr int ROW_SLOTS = IMG ? IMG_DMA : 2 * PRE_TDMA;
+    uint32_t doff[SPW];
+    bool dlive[SPW];
 #pragma unroll
-    for (int s = 0; s < PRE_SPW; s++) {
+    for (int s = 0; s < SPW; s++) {
         const int slot = wave + PRE_WAVES * s;
         uint32_t off = 0;
         bool live = false;
-        if (slot < 2 * PRE_TDMA) {
+        if (IMG && slot < ROW_SLOTS) {
+            off = (uint32_t) (slot * 1024 + lane * 16);
+            live = true;
+        } else if (slot < ROW_SLOTS) {
             const int tensor = slot >= PRE_TDMA;
             const uint32_t p = (uint32_t) ((slot - tensor * PRE_TDMA) * 64 + lane), key = p / 17u, part = p - key * 17u;
             off = key * (uint32_t) (tensor ? a.v_nb1 : a.k_nb1) + part * 16u;
             live = true;
-        } else if (MASKED && slot < PRE_SLOTS && slot - 2 * PRE_TDMA < n_mdma) {
-            const int g = (slot - 2 * PRE_TDMA) * 64 + lane;
+        } else if (MASKED && slot < ROW_SLOTS + PRE_MDMA && slot - ROW_SLOTS < n_mdma) {
+            const int g = (slot - ROW_SLOTS) * 64 + lane;
             const int gc = g < n_mrows * PRE_MGR ? g : n_mrows * PRE_MGR - 1;
             off = (mrow_off(gc / PRE_MGR) & ~15u) + 16u * (uint32_t) (gc % PRE_MGR);
             live = true;
@@ -4210,23 +4355,24 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
     auto issue_chunk = [&](int c, uint8_t * st) __attribute__((always_inline)) {
         const int64_t c0 = k_lo + (int64_t) c * PRE_CK;
         const int64_t kc = c0 * (int64_t) a.k_nb1, vc = c0 * (int64_t) a.v_nb1;
-        const v4i rk = make_rsrc(kbase + kc, (uint32_t) std::min<int64_t>(k_bytes - kc, 0xffffffffll));
-        const v4i rv = make_rsrc(vbase + vc, (uint32_t) std::min<int64_t>(v_bytes - vc, 0xffffffffll));
+        const v4i rk = IMG ? make_rsrc(a.img + ((size_t) kvh * a.img_chunks + (size_t) (c0 / PRE_CK)) * IMG_BYTES, IMG_BYTES)
+                           : make_rsrc(kbase + kc, (uint32_t) std::min<int64_t>(k_bytes - kc, 0xffffffffll));
+        const v4i rv = IMG ? rk : make_rsrc(vbase + vc, (uint32_t) std::min<int64_t>(v_bytes - vc, 0xffffffffll));
         v4i rm = rk;
         if constexpr (MASKED)
             rm = make_rsrc(mslice_al + c0 * 2, (uint32_t) (a.m_slice + (uint32_t) (mslice - mslice_al) - c0 * 2));
 #pragma unroll
-        for (int s = 0; s < PRE_SPW; s++) {
+        for (int s = 0; s < SPW; s++) {
             const int slot = wave + PRE_WAVES * s;
             if (!dlive[s]) continue;
-            dma16_buf(slot < PRE_TDMA ? rk : slot < 2 * PRE_TDMA ? rv : rm, doff[s],
+            dma16_buf(slot >= ROW_SLOTS ? rm : IMG || slot < PRE_TDMA ? rk : rv, doff[s],
                       __builtin_amdgcn_readfirstlane(lds_addr(st + slot * 1024)));
         }
     };
     // fused append (as in k_fa_dec): the blocks whose keys hold appended rows
     // quantise their KV head's part of them first, and their chunk DMAs read
     // the rows only after these stores are done
-    if (a.app_n > 0) {
+    if (!IMG && a.app_n > 0) {
         const int64_t alo = std::max<int64_t>(a.app_row0, k_lo), ahi = std::min<int64_t>(a.app_row0 + a.app_n, k_hi);
         if (alo < ahi) {
             const int units = (int) (ahi - alo) * NBLK * 2;
@@ -4260,7 +4406,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
     // ---- prologue: each wave requantises its own 16 query rows (ggml's
     //      quantiser; 4 lanes per (row, block)) into an image of its own, from
     //      which lane (ln, lg) takes quants 8 lg .. 8 lg + 7 of each block of row ln ----
-    uint8_t * qimg = lds + wave * PRE_QW;                   // [block][row][32] int8
+    uint8_t * qimg = lds + (IMG ? STAGE : 0) + wave * PRE_QW;   // [block][row][32] int8
     float * dql = (float *) (qimg + PRE_QIMG);                  // [16 rows][NBLK]
     long qw[NBLK];
     float dq[NBLK];
@@ -4307,7 +4453,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
     // row's offset within its first granule
     const int rl_lane = wr0 + ln < RW ? wr0 + ln : 0;
     const int mrow = MASKED ? (int) div_gqa(a, (uint32_t) (r0 + rl_lane)) - t0 : 0;
-    const uint32_t m_lane = MASKED ? (uint32_t) (PRE_MOFF + mrow * PRE_MGR * 16) + (mrow_off(mrow) & 15u) + 8u * (uint32_t) lg : 0u;
+    const uint32_t m_lane = MASKED ? (uint32_t) (MOFF + mrow * PRE_MGR * 16) + (mrow_off(mrow) & 15u) + 8u * (uint32_t) lg : 0u;
     const bool wave_rows = wr0 < RW;   // the wave has rows of its own
 
     v4f O[NBLK][2];
@@ -4318,71 +4464,17 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
     // ---- the key loop: chunk c in stage c % 2; chunk c + 1 loads while chunk c
     //      is converted and computed ----
     for (int c = 0; c < n_chunks; c++) {
-        uint8_t * st = stg + (c & 1) * PRE_STAGE;
+        uint8_t * st = stg + (c & 1) * STAGE;
+        uint8_t * const vt = IMG ? st : lds, * const kq = vt + (IMG ? IMG_K : PRE_VT);
+        uint16_t (* const skv)[NBLK][PRE_CK] =
+            (uint16_t (*)[NBLK][PRE_CK]) (vt + (IMG ? IMG_S : PRE_VT + PRE_KQ));   // [K|V][block][key] fp16 scales
         wait_vmcnt<0>();
         __syncthreads();   // chunk c has landed; every wave is done with chunk c - 1 (and the prologue)
-        if (c + 1 < n_chunks) issue_chunk(c + 1, stg + ((c + 1) & 1) * PRE_STAGE);
-        // conversion pass: wave w takes V block w (dims 32w .. 32w+31) of the
-        // 64 keys: lane (key pair kp, half dh) converts dims 32w + 16dh .. +15 of
-        // the keys at V^T positions 2kp, 2kp + 1, and K block w of key `lane`
-        // into the repacked quants; lane k also tabulates the K and V scales of
-        // block w of key k. Block w's quants start 2 bytes into a word when w
-        // is even and on a word boundary when w is odd (34w + 2 = 0 mod 4): the
-        // lanes read whole words from the word at or before them and realign
-        // them with alignbyte (shift 2 or 0), with no branch on the parity.
-        // Rows sit 272 bytes (68 words, 4 banks mod 32) apart, so reads of one
-        // offset in many rows would meet in 8 banks: each lane reads its run of
-        // words starting at a rotated word (slot i holds word (i + rot) mod n,
-        // the word past the run sits in slot n), so that one read's lanes cover
-        // every bank. Every read is issued before the first conversion.
-        {
-            const int kp = lane & 31, dh = lane >> 5;
-            const int p0 = 2 * kp;
-            // the key at position p0 (its neighbour p0 + 1 is the next key)
-            const int key0 = 32 * (p0 >> 5) + 16 * ((p0 >> 2) & 1) + 4 * ((p0 >> 3) & 3) + (p0 & 3);
-            const int odd = wave & 1;
-            const uint32_t sh = odd ? 0u : 2u;
-            const uint8_t * v0 = st + PRE_KB + key0 * SEG + QBLOCK * wave + 16 * dh + 2 * odd;
-            const uint8_t * k0 = st + lane * SEG + QBLOCK * wave + 2 * odd;
-            const int vrot = (kp >> 3) & 3, krot = (lane >> 3) & 7;
-            uint32_t x[5], y[5], kw[9];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int t = (i + vrot) & 3;
-                x[i] = *(const uint32_t *) (v0 + 4 * t);
-                y[i] = *(const uint32_t *) (v0 + SEG + 4 * t);
-            }
-            x[4] = *(const uint32_t *) (v0 + 16);
-            y[4] = *(const uint32_t *) (v0 + SEG + 16);
-#pragma unroll
-            for (int i = 0; i < 8; i++) kw[i] = *(const uint32_t *) (k0 + 4 * ((i + krot) & 7));
-            kw[8] = *(const uint32_t *) (k0 + 32);
-            const uint16_t dk16 = *(const uint16_t *) (st + lane * SEG + QBLOCK * wave);
-            const uint16_t dv16 = *(const uint16_t *) (st + PRE_KB + lane * SEG + QBLOCK * wave);
-            // V: word t of the lane's 16 bytes holds dims 16dh + 4t .. + 3 of keys key0 / key0 + 1
-            uint8_t * vrow = vt + (32 * wave + 16 * dh) * PRE_VTS + 2 * p0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int t = (i + vrot) & 3;
-                const uint32_t xa = __builtin_amdgcn_alignbyte(t == 3 ? x[4] : x[(i + 1) & 3], x[i], sh);
-                const uint32_t ya = __builtin_amdgcn_alignbyte(t == 3 ? y[4] : y[(i + 1) & 3], y[i], sh);
-                uint8_t * d = vrow + 4 * t * PRE_VTS;
-                *(uint32_t *) (d) = cvt_i8_pair<0>(xa, ya);
-                *(uint32_t *) (d + PRE_VTS) = cvt_i8_pair<1>(xa, ya);
-                *(uint32_t *) (d + 2 * PRE_VTS) = cvt_i8_pair<2>(xa, ya);
-                *(uint32_t *) (d + 3 * PRE_VTS) = cvt_i8_pair<3>(xa, ya);
-            }
-            // K: word j of block w of key `lane` (quants 4j .. 4j + 3) to kq[w][lane]
-            uint8_t * kd = kq + (wave * PRE_CK + lane) * PRE_KQS;
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int t = (i + krot) & 7;
-                *(uint32_t *) (kd + 4 * t) = __builtin_amdgcn_alignbyte(t == 7 ? kw[8] : kw[(i + 1) & 7], kw[i], sh);
-            }
-            skv[0][wave][lane] = dk16;
-            skv[1][wave][lane] = dv16;
+        if (c + 1 < n_chunks) issue_chunk(c + 1, stg + ((c + 1) & 1) * STAGE);
+        if constexpr (!IMG) {
+            pre_convert<false>(st, vt, kq, skv, lane, wave);
+            __syncthreads();   // V^T and the scale tables of chunk c are complete
         }
-        __syncthreads();   // V^T and the scale tables of chunk c are complete
 
         // ---- the wave's 16 rows over the chunk's keys: the lane's keys are
         //      16 kt + 4 lg + i (key tile kt, i = 0..3) ----
@@ -4417,10 +4509,10 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
             long kA[2][NBLK];
             uint2 dk[2][NBLK];
             auto load_tile = [&](int kt, long (&ka)[NBLK], uint2 (&dkk)[NBLK]) __attribute__((always_inline)) {
-                const uint8_t * kr = kq + (16 * kt + ln) * PRE_KQS + 8 * lg;
+                const uint8_t * kr = kq + (16 * kt + ln) * KQS + 8 * (IMG ? lg ^ (ln >> 2) : lg);
 #pragma unroll
                 for (int bb = 0; bb < NBLK; bb++) {
-                    ka[bb] = *(const long *) (kr + bb * PRE_CK * PRE_KQS);
+                    ka[bb] = *(const long *) (kr + bb * PRE_CK * KQS);
                     dkk[bb] = *(const uint2 *) &skv[0][bb][16 * kt + 4 * lg];
                 }
             };
@@ -4514,9 +4606,10 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
             v8h Bh[2], Bl[2];
             auto load_a = [&](int n, v8h (&aa)[2]) __attribute__((always_inline)) {
                 const int h = n >> 3, bb = n & 7;
-                const uint8_t * va = vt + (32 * bb + ln) * PRE_VTS + (32 * h + 8 * lg) * 2;
+                constexpr int VS = IMG ? IMG_VS : PRE_VTS;
+                const uint8_t * va = vt + (32 * bb + ln) * VS + (IMG ? 16 * ((4 * h + lg) ^ (2 * (ln & 3))) : (32 * h + 8 * lg) * 2);
                 aa[0] = *(const v8h *) va;
-                aa[1] = *(const v8h *) (va + 16 * PRE_VTS);
+                aa[1] = *(const v8h *) (va + 16 * VS);
             };
             auto load_dv = [&](int n, uint2 (&dd)[2]) __attribute__((always_inline)) {
                 const int h = n >> 3, bb = n & 7;
@@ -4630,7 +4723,9 @@ struct fa_plan {
     int32_t pre_rgmap;                // k_fa_pre block order (fa_args::pre_rgmap)
     fa_kind kind;
     size_t  off_ml;                   // workspace section of the split (max, sum) pairs (bytes)
-    size_t  ws_bytes;
+    size_t  ws_base;                  // bytes the split partials need
+    size_t  ws_bytes;                 // with the chunk images behind them, where the plan has them
+    int32_t img_chunks;               // k_fa_pre: chunks whose images are made first (0: none)
     // per-sequence key counts: splits of each sequence (ns is the largest)
     int32_t ragged;
     int32_t r_ustart[RAGGED_MAX_B + 1], r_ns[RAGGED_MAX_B], r_split_len[RAGGED_MAX_B];
@@ -4729,6 +4824,7 @@ int check_no_scratch() {
                                (const void *) k_fa_vs<1, 1, false, true, false>, (const void *) k_fa_vs<1, 1, true, true, false>,
                                (const void *) k_fa_vs<1, 1, false, false, true>,
                                (const void *) k_fa_pre<false>, (const void *) k_fa_pre<true>,
+                               (const void *) k_fa_pre<false, true>, (const void *) k_fa_pre<true, true>,
                                (const void *) k_fa_qc<2>, (const void *) k_fa_qc<4>, (const void *) k_fa_qc<8>,
                                (const void *) k_fattn_q8_0<2, true, WAVES, 16, false>,
                                (const void *) k_fattn_q8_0<1, false, WAVES_PAIR, 16, false>,
@@ -4750,6 +4846,16 @@ int check_no_scratch() {
     }();
     if (rc) set_error(rc, "flash_attn_ext: attention kernel uses scratch memory (build is unusable)");
     return rc;
+}
+
+// Whether k_fa_pre's chunks are converted to images first: where a block walks
+// enough chunks to win the image launch back and enough row groups share a
+// chunk to win its bytes back. Attention op without and with images, 2 KV
+// heads: 33 chunks a block, 64 row groups 380 -> 328 us; 24 (48 x 2 row groups)
+// 272 -> 235; 11.5 (6) 167 -> 155; 9.5 (38) 142 -> 130; but 8.4 (16) 73.3 ->
+// 74.0; 6 (32) 58.1 -> 59.0; 2 (32) 34.8 -> 37.1.
+bool pre_images(int64_t B, int64_t n_rg, int64_t split_chunks) {
+    return B == 1 && n_rg >= 6 && split_chunks >= 9;
 }
 
 int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v, const qwfn_tensor * mask,
@@ -4882,9 +4988,13 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         size_t off = align256(n_part * D * sizeof(float));
         pl->off_ml = off;
         off = align256(off + n_part * sizeof(float2));
-        pl->ws_bytes = std::max<size_t>(off, 256);
+        pl->ws_base = pl->ws_bytes = std::max<size_t>(off, 256);
+        const int64_t chunks = (n_kv + PRE_CK - 1) / PRE_CK;
+        pl->img_chunks = pre_images(B, pl->n_rg, split_len / PRE_CK) ? (int32_t) chunks : 0;
+        if (pl->img_chunks) pl->ws_bytes += (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
         return QWFN_OK;
     }
+    pl->img_chunks = 0;
     const bool vs = pl->kind == FA_VS;
     const bool vd = pl->kind == FA_VD || vs, kdec = pl->kind == FA_DEC;
     pl->R = (int32_t) R;
@@ -5015,7 +5125,7 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
     size_t off = align256(n_part * D * sizeof(float));
     pl->off_ml = off;
     off = align256(off + n_part * sizeof(float2));
-    pl->ws_bytes = std::max<size_t>(off, 256);
+    pl->ws_base = pl->ws_bytes = std::max<size_t>(off, 256);
     return QWFN_OK;
 }
 
@@ -5156,12 +5266,12 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
     if (variant != QWFN_Q8_REF && variant != QWFN_Q8_X86) return set_error(QWFN_EINVAL, "flash_attn_ext: unknown variant");
     fa_plan pl{};
     if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, MAX_SPLITS, gat != nullptr)) return rc;
-    if (wsm == WS_SCRATCH && pl.ws_bytes > NOALLOC_SCRATCH_BYTES) {
+    if (wsm == WS_SCRATCH && pl.ws_base > NOALLOC_SCRATCH_BYTES) {
         // fewer key splits, so that their partials fit the scratch
         const size_t per_split = (size_t) q->ne[3] * k->ne[2] * pl.R * (D * sizeof(float) + sizeof(float2));
         const int64_t cap = std::max<int64_t>(1, (int64_t) ((NOALLOC_SCRATCH_BYTES - 512) / std::max<size_t>(per_split, 1)));
         if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, cap, gat != nullptr)) return rc;
-        if (pl.ws_bytes > NOALLOC_SCRATCH_BYTES)
+        if (pl.ws_base > NOALLOC_SCRATCH_BYTES)
             return set_error(QWFN_ENOMEM, "flash_attn_ext_noalloc: the split partials need more than the 16 MiB scratch");
     }
     if (app)
@@ -5182,6 +5292,12 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
         hipLaunchKernelGGL(k_zero_f32, dim3((unsigned) std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 4096))),
                            dim3(256), 0, as_stream(stream), (float *) dst->data, n);
         return hip_check(hipGetLastError(), "flash_attn zero fill");
+    }
+    // no images where the workspace holds the partials only, or with rows that
+    // the attention kernel itself appends
+    if (app || (wsm == WS_SCRATCH ? NOALLOC_SCRATCH_BYTES : ws ? ws_bytes : pl.ws_bytes) < pl.ws_bytes) {
+        pl.img_chunks = 0;
+        pl.ws_bytes = pl.ws_base;
     }
     if (wsm == WS_SCRATCH) {
         if (int rc = scratch_address(&ws)) return rc;
@@ -5274,8 +5390,18 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
         a.nrg_mul = recip32(a.n_rg);
         a.nbh_mul = recip32(a.B * a.nh_kv);
         const dim3 g((unsigned) grid), bd(PRE_WAVES * 64);
-        if (a.mask) QWFN_FA_LAUNCH(g, bd, as_stream(stream), k_fa_pre<true>);
-        else        QWFN_FA_LAUNCH(g, bd, as_stream(stream), k_fa_pre<false>);
+        if (pl.img_chunks) {
+            a.img = (uint8_t *) w + pl.ws_base;
+            a.img_chunks = pl.img_chunks;
+            hipLaunchKernelGGL(k_fa_pre_image, dim3((unsigned) pl.img_chunks, (unsigned) a.nh_kv), bd, 0, as_stream(stream), a);
+            if (int rc = hip_check(hipGetLastError(), "flash_attn image launch")) return rc;
+            if (a.mask) QWFN_FA_LAUNCH(g, bd, as_stream(stream), k_fa_pre<true, true>);
+            else        QWFN_FA_LAUNCH(g, bd, as_stream(stream), k_fa_pre<false, true>);
+        } else if (a.mask) {
+            QWFN_FA_LAUNCH(g, bd, as_stream(stream), k_fa_pre<true>);
+        } else {
+            QWFN_FA_LAUNCH(g, bd, as_stream(stream), k_fa_pre<false>);
+        }
         g_last_merge = a.ns > 1 ? QWFN_FA_MERGE_KERNEL : QWFN_FA_MERGE_NONE;
         if (int rc = hip_check(hipGetLastError(), "flash_attn launch")) return rc;
         if (a.ns > 1) {
