@@ -4858,6 +4858,48 @@ bool pre_images(int64_t B, int64_t n_rg, int64_t split_chunks) {
     return B == 1 && n_rg >= 6 && split_chunks >= 9;
 }
 
+// The time of a k_fa_pre call of ns key splits in a block order (fa_args::
+// pre_rgmap), in us: an XCD's blocks run in rounds of its 32 CUs, each as long
+// as a block's chunks (5 us from images, else 6) and its prologue and epilogue
+// (6); the partials are written and read back, and the bytes the XCDs' L2s
+// cannot share (the f32 query rows once per split where units share an XCD, the
+// K/V rows once per XCD holding a KV head's row groups where splits do) come
+// again, at 4 TB/s. Measured where it decides (splits: us): 48 row groups, 72
+// chunks 3: 243, 4: 204, 5: 180, 6: 218, 8: 187; 38 row groups, 38 chunks 3: 93,
+// 4: 131; 19, 69 chunks 6: 88, 7: 117; 29, 133 chunks 4: 193, 5: 250.
+// (32-bit and shifts: a call evaluates up to 256 split counts)
+float pre_cost(uint32_t nbh, uint32_t n_rg, uint32_t chunks, float part, float q_rep, float kv_rep, uint32_t ns, bool * rgmap) {
+    const uint32_t sc = (chunks + ns - 1) / ns;
+    const float block = (float) sc * (pre_images(1, n_rg, sc) ? 5.f : 6.f) + 6.f;
+    const uint32_t units = (nbh * ns + 7) >> 3, rgus = (nbh * n_rg + 7) >> 3;
+    const float c0 = (float) ((n_rg * units + 31) >> 5) * block + q_rep * (float) (ns - 1);
+    const float c1 = (float) ((ns * rgus + 31) >> 5) * block + kv_rep;
+    *rgmap = ns > 1 && c1 < c0;
+    return (*rgmap ? c1 : c0) + (ns > 1 ? part * (float) ns + 4.f : 0.f);
+}
+
+// k_fa_pre's key splits and block order: the cheapest count of whole chunks, at
+// least two a split, within three rounds of blocks (one where a call has few
+// row groups); forced: that count
+int64_t pre_splits(int64_t nbh, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced, bool * rgmap) {
+    const int64_t chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK), per = nbh * n_rg;
+    *rgmap = false;
+    // (beyond 32 bits: more blocks than any split count is needed for)
+    if (per >= (int64_t(1) << 24) || chunks >= (int64_t(1) << 24)) return forced ? std::min(forced, ns_cap) : 1;
+    const float part = 2.f * (float) (R * nbh) * D * 4 / 4e6f, q_rep = (float) R * D * 4 / 4e6f;
+    const float kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
+    const int64_t most = std::min<int64_t>({(chunks + 1) / 2, ns_cap, std::max<int64_t>(1, (per < 8 ? 256 : 768) / per)});
+    const int64_t lo = forced ? std::max<int64_t>(1, std::min(forced, ns_cap)) : 1, hi = forced ? lo : std::max<int64_t>(1, most);
+    int64_t best = lo;
+    float cost = INFINITY;
+    for (int64_t n = lo; n <= hi; n++) {
+        bool m;
+        const float c = pre_cost((uint32_t) nbh, (uint32_t) n_rg, (uint32_t) chunks, part, q_rep, kv_rep, (uint32_t) n, &m);
+        if (c < cost) { cost = c; best = n; *rgmap = m; }
+    }
+    return best;
+}
+
 int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v, const qwfn_tensor * mask,
                fa_plan * pl, const int64_t * seq_n_kv = nullptr, int64_t ns_cap = MAX_SPLITS, bool gather = false) {
     if (!q || !k || !v) return set_error(QWFN_EINVAL, "flash_attn_ext: NULL q/k/v");
@@ -4953,22 +4995,17 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
     if (vd_ok && fk == QWFN_FA_KERNEL_AUTO && R <= 8 && B == 1 && !seq_n_kv && !gather && n_kv <= VS_AUTO_MAX_KEYS)
         pl->kind = FA_VS;
     if (pre_ok && (fk == QWFN_FA_KERNEL_AUTO || fk == QWFN_FA_KERNEL_PRE)) {
-        // k_fa_pre: 128-row blocks; key splits of whole 64-key chunks (at least
-        // two per split), about one block per CU; the row groups of a (batch,
-        // KV head, split) unit share an XCD
+        // k_fa_pre: 128-row blocks; key splits of whole 64-key chunks
         pl->kind = FA_PRE;
         pl->R = (int32_t) R;
         pl->rw = PRE_ROWS;
         pl->RT = PRE_WAVES;
         pl->n_rg = (int32_t) ((R + PRE_ROWS - 1) / PRE_ROWS);
         pl->gqa = (int32_t) gqa;
-        const int64_t per = nh_kv * B * pl->n_rg;
-        int64_t ns = std::max<int64_t>(1, (256 + per - 1) / per);
-        ns = std::min<int64_t>(ns, std::max<int64_t>(1, n_kv / (2 * PRE_CK)));
-        if (const int32_t force = g_force_splits.load(std::memory_order_relaxed)) ns = force;
-        ns = std::max<int64_t>(1, std::min<int64_t>(ns, ns_cap));
-        int64_t split_len = (n_kv + ns - 1) / ns;
-        split_len = std::max<int64_t>(PRE_CK, (split_len + PRE_CK - 1) / PRE_CK * PRE_CK);
+        const int64_t chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK);
+        bool rgmap;
+        int64_t ns = pre_splits(B * nh_kv, pl->n_rg, R, n_kv, ns_cap, g_force_splits.load(std::memory_order_relaxed), &rgmap);
+        const int64_t split_len = (chunks + ns - 1) / ns * PRE_CK;
         ns = std::max<int64_t>(1, (n_kv + split_len - 1) / split_len);
         if (ns > MAX_SPLITS)
             return set_error(QWFN_ENOTSUP, "flash_attn_ext: " + std::to_string(ns) + " key splits requested, at most " +
@@ -4977,19 +5014,12 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         pl->split_len = (int32_t) split_len;
         pl->max_span = split_len;
         pl->ragged = 0;
-        // block order: the bytes an XCD's L2 cannot share. Units on an XCD read
-        // each KV head's f32 query rows once per split; row groups on an XCD
-        // (one KV head an XCD) read its K/V rows once per XCD holding its rows
-        const int64_t nbh = B * nh_kv;
-        const double q_rep = (double) R * D * 4 * (double) (ns - 1);
-        const double kv_rep = (double) n_kv * (2.0 * (D / 32) * 34) * (double) (std::max<int64_t>(1, 8 / nbh) - 1);
-        pl->pre_rgmap = ns > 1 && q_rep > kv_rep ? 1 : 0;
+        pl->pre_rgmap = ns > 1 && rgmap;
         const size_t n_part = ns > 1 ? (size_t) (B * nh_kv * ns * R) : 0;
         size_t off = align256(n_part * D * sizeof(float));
         pl->off_ml = off;
         off = align256(off + n_part * sizeof(float2));
         pl->ws_base = pl->ws_bytes = std::max<size_t>(off, 256);
-        const int64_t chunks = (n_kv + PRE_CK - 1) / PRE_CK;
         pl->img_chunks = pre_images(B, pl->n_rg, split_len / PRE_CK) ? (int32_t) chunks : 0;
         if (pl->img_chunks) pl->ws_bytes += (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
         return QWFN_OK;
