@@ -305,6 +305,11 @@ __device__ __forceinline__ float sum_lanes16_32(float x) {
     return reduce_lanes16_32(x, [](float a, float b) { return a + b; });
 }
 
+// x of the lane 8 away in the row of 16
+__device__ __forceinline__ float ror8(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xf, 0xf, false));
+}
+
 // s_waitcnt that waits for vmcnt <= n only (gfx9 encoding: vmcnt[3:0] in
 // bits 3:0, vmcnt[5:4] in bits 15:14, expcnt and lgkmcnt left at their max).
 template <int N>
@@ -2070,7 +2075,7 @@ __global__ __launch_bounds__(DEC_WAVES * 64, 2) void k_fa_dec(fa_args a) {
 
 // ================================================================ many per-position cell lists
 //
-// k_fa_qc<KG> (KG = 2, 4, 8): attention of many query positions, each over its own list of
+// k_fa_qc<KG, PK> (KG = 2, 4, 8): attention of many query positions, each over its own list of
 // cache cells (the keys a query of a QSA-on prefill chunk sees: its selected
 // cells at or before its position, qwfn_graph.cpp:388-414 and :466-471), with
 // the list lengths on the device. A unit is one (position, KV head) list and
@@ -2083,6 +2088,19 @@ __global__ __launch_bounds__(DEC_WAVES * 64, 2) void k_fa_dec(fa_args a) {
 // merge in LDS and the unit's rows go straight to dst (times sigmoid(gate)).
 // Blocks alternate over the KV heads, so with 2 KV heads each XCD's L2 serves
 // one head's rows.
+//
+// The key loop is bound by the vector unit (scaling of the block dots, the V
+// rows' conversion, P*d_v's split), and with at most 8 rows half of a tile's 16
+// columns repeat zeros. PK (n_head / n_head_kv <= 8) puts two things in one
+// tile instead: K*Q of an even block in columns 0 .. 7 and of the odd block
+// after it in 8 .. 15 (the other half of each operand is zero, so the second
+// MFMA adds to the first; one scaling serves both blocks), and P*d_v's hi part
+// in columns 0 .. 7, its lo part in 8 .. 15 (one MFMA for both). The scores'
+// halves meet at each tile, the outputs' once after the last. 512 positions at
+// 16384 (16 heads on 2, 1024 cells each): 140 -> 129 us, the error against 64
+// bits as it was (3.1e-6). From 9 rows on the plain form is the only one. The
+// same packing in k_fa_dec measured nothing (four sequences of 8K .. 64K: 36.4
+// us either way): there the wait is for the rows, not for the vector unit.
 //
 // The tile's cells come by LDS DMA too, into four slots per wave, so every
 // vector-memory load of the key loop is a DMA and the explicit counts stay
@@ -2118,7 +2136,7 @@ struct qc_args {
     uint32_t *      status;
 };
 
-template <int KG>
+template <int KG, bool PK>
 __global__ __launch_bounds__(QC_WAVES * 64, 1) void k_fa_qc(qc_args a) {
     constexpr int UPB = QC_WAVES / KG;                 // units of a block
     constexpr int QR = 16 * UPB;                       // query rows staged by the block
@@ -2275,15 +2293,20 @@ __global__ __launch_bounds__(QC_WAVES * 64, 1) void k_fa_qc(qc_args a) {
                   win_off(5) == 12 && win_off(6) == 14 && win_off(7) == 32, "the packed window offsets");
     __syncthreads();
     const int rl_lane = unit * 16 + ln;
+    // PK: an even block's operand is zero in columns 8 .. 15 (its rows past the
+    // group), an odd one's holds the rows there instead; dq: the column's blocks
+    constexpr int NDQ = PK ? NBLK / 2 : NBLK;
+    const int hi8 = ln >> 3;
     v4i qw[NBLK];
-    float dq[NBLK];
+    float dq[NDQ];
 #pragma unroll
-    for (int bb = 0; bb < NBLK; bb++) {
-        qw[bb] = *(const v4i *) qslice(bb, lg, rl_lane);
-        dq[bb] = dql[rl_lane * NBLK + bb];
-    }
+    for (int bb = 0; bb < NBLK; bb++) qw[bb] = *(const v4i *) qslice(bb, lg, PK && (bb & 1) ? rl_lane ^ 8 : rl_lane);
 #pragma unroll
-    for (int bb = 0; bb < NBLK; bb++) asm volatile("" : "+v"(qw[bb]), "+v"(dq[bb]));
+    for (int bb = 0; bb < NDQ; bb++) dq[bb] = PK ? dql[(unit * 16 + (ln & 7)) * NBLK + 2 * bb + hi8] : dql[rl_lane * NBLK + bb];
+#pragma unroll
+    for (int bb = 0; bb < NBLK; bb++) asm volatile("" : "+v"(qw[bb]));
+#pragma unroll
+    for (int bb = 0; bb < NDQ; bb++) asm volatile("" : "+v"(dq[bb]));
     __syncthreads();   // every wave has its operands: stage 1 is free
     // the order of a steady step (tile 0's V rows, then tile 2's cells, tile
     // 1's K and V, tile 3's cells): tiles 2 and 3's cells are already in
@@ -2316,7 +2339,30 @@ __global__ __launch_bounds__(QC_WAVES * 64, 1) void k_fa_qc(qc_args a) {
         }
         wave_lds_sync();
         float s[4] = {0.f, 0.f, 0.f, 0.f};
-        {
+        if constexpr (PK) {
+            v4i kA[NBLK];
+            uint2 dk[NDQ];
+            const uint8_t * krow = st + ln * SEG + 16 * lg;
+#pragma unroll
+            for (int bb = 0; bb < NBLK; bb++) kA[bb] = *(const v4i *) (krow + 16 * win_piece(bb));
+#pragma unroll
+            for (int pp = 0; pp < NDQ; pp++) dk[pp] = *(const uint2 *) &sw[0][2 * pp + hi8][lg * 4];
+            v4i cc[NDQ];
+#pragma unroll
+            for (int pp = 0; pp < NDQ; pp++) cc[pp] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kA[2 * pp], qw[2 * pp], v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+            for (int pp = 0; pp < NDQ; pp++) cc[pp] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kA[2 * pp + 1], qw[2 * pp + 1], cc[pp], 0, 0, 0);
+#pragma unroll
+            for (int pp = 0; pp < NDQ; pp++) {
+                const float d = dq[pp];
+                s[0] = __builtin_fmaf((float) cc[pp][0], mul_f16lo(d, dk[pp].x), s[0]);
+                s[1] = __builtin_fmaf((float) cc[pp][1], mul_f16hi(d, dk[pp].x), s[1]);
+                s[2] = __builtin_fmaf((float) cc[pp][2], mul_f16lo(d, dk[pp].y), s[2]);
+                s[3] = __builtin_fmaf((float) cc[pp][3], mul_f16hi(d, dk[pp].y), s[3]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[i] += ror8(s[i]);
+        } else {
             v4i kA[NBLK];
             uint2 dk[NBLK];
             const uint8_t * krow = st + ln * SEG + 16 * lg;
@@ -2403,15 +2449,19 @@ __global__ __launch_bounds__(QC_WAVES * 64, 1) void k_fa_qc(qc_args a) {
             const v4h A1 = __builtin_bit_cast(v4h, make_uint2(a1[0], a1[1]));
             const v4h Bh = __builtin_bit_cast(v4h, make_uint2(bh[0], bh[1]));
             const v4h Bl = __builtin_bit_cast(v4h, make_uint2(bl[0], bl[1]));
-            O[bb][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, Bh, O[bb][0], 0, 0, 0);
-            O[bb][1] = __builtin_amdgcn_mfma_f32_16x16x16f16(A1, Bh, O[bb][1], 0, 0, 0);
+            // PK: P*d_v's hi part in columns 0 .. 7, its lo part in the same rows' columns 8 .. 15
+            const v4h B = PK ? __builtin_bit_cast(v4h, make_uint2(hi8 ? bl[0] : bh[0], hi8 ? bl[1] : bh[1])) : Bh;
+            O[bb][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, B, O[bb][0], 0, 0, 0);
+            O[bb][1] = __builtin_amdgcn_mfma_f32_16x16x16f16(A1, B, O[bb][1], 0, 0, 0);
             if (bb + 1 < NBLK) {
                 const uint32_t dv[2] = {dv2[bb + 1].x, dv2[bb + 1].y};
                 cvt_v_block(w[bb + 1], a0, a1);
                 pdv_hilo(p, p16, dv, bh, bl);
             }
-            O[bb][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, Bl, O[bb][0], 0, 0, 0);
-            O[bb][1] = __builtin_amdgcn_mfma_f32_16x16x16f16(A1, Bl, O[bb][1], 0, 0, 0);
+            if constexpr (!PK) {
+                O[bb][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, Bl, O[bb][0], 0, 0, 0);
+                O[bb][1] = __builtin_amdgcn_mfma_f32_16x16x16f16(A1, Bl, O[bb][1], 0, 0, 0);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
         issue_v(stl);                  // the rows issue_k(j + 2) read
@@ -2433,6 +2483,13 @@ __global__ __launch_bounds__(QC_WAVES * 64, 1) void k_fa_qc(qc_args a) {
     }
     __builtin_amdgcn_s_setprio(0);
     wait_vmcnt<0>();   // every DMA of the wave has landed (those past the list included)
+
+    if constexpr (PK) {                // the hi and the lo columns of a row
+#pragma unroll
+        for (int bb = 0; bb < NBLK; bb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) { O[bb][0][i] += ror8(O[bb][0][i]); O[bb][1][i] += ror8(O[bb][1][i]); }
+    }
 
     // ---- merge the KG waves of each unit ----
     {
@@ -4825,7 +4882,8 @@ int check_no_scratch() {
                                (const void *) k_fa_vs<1, 1, false, false, true>,
                                (const void *) k_fa_pre<false>, (const void *) k_fa_pre<true>,
                                (const void *) k_fa_pre<false, true>, (const void *) k_fa_pre<true, true>,
-                               (const void *) k_fa_qc<2>, (const void *) k_fa_qc<4>, (const void *) k_fa_qc<8>,
+                               (const void *) k_fa_qc<2, false>, (const void *) k_fa_qc<4, false>, (const void *) k_fa_qc<8, false>,
+                               (const void *) k_fa_qc<2, true>, (const void *) k_fa_qc<4, true>, (const void *) k_fa_qc<8, true>,
                                (const void *) k_fattn_q8_0<2, true, WAVES, 16, false>,
                                (const void *) k_fattn_q8_0<1, false, WAVES_PAIR, 16, false>,
                                (const void *) k_fattn_q8_0<1, true, WAVES_PAIR, 16, false>,
@@ -5768,7 +5826,8 @@ extern "C" int qwfn_flash_attn_ext_q8_0_query_cells_dev(const qwfn_tensor * q, c
         const int64_t upb = QC_WAVES / kg;
         const int64_t blocks = (T + upb - 1) / upb * nh_kv;
         if (blocks > INT32_MAX) return fail(QWFN_ENOTSUP, "too many positions");
-        auto kern = kg == 2 ? k_fa_qc<2> : kg == 4 ? k_fa_qc<4> : k_fa_qc<8>;
+        auto kern = a.gqa <= 8 ? (kg == 2 ? k_fa_qc<2, true> : kg == 4 ? k_fa_qc<4, true> : k_fa_qc<8, true>)
+                               : (kg == 2 ? k_fa_qc<2, false> : kg == 4 ? k_fa_qc<4, false> : k_fa_qc<8, false>);
         hipLaunchKernelGGL(kern, dim3((unsigned) blocks), dim3(QC_WAVES * 64), 0, as_stream(stream), a);
         return hip_check(hipGetLastError(), "flash_attn_ext_query_cells_dev launch");
     });
