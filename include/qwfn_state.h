@@ -222,7 +222,8 @@ int qwfn_qsa_select_cells(const uint16_t * pool, size_t pool_nb1, int64_t n_bloc
 /* ------------------------------------------------- Gated DeltaNet state */
 
 /* The recurrent update of a DeltaNet layer for T tokens with its rollback
- * snapshots, one launch: ggml_gated_delta_net (qwfn_graph.cpp:258, inside
+ * snapshots, one launch (two where 12 or more tokens come before the last
+ * n_snap + 1 of a call with snapshots): ggml_gated_delta_net (qwfn_graph.cpp:258, inside
  * graph_builder::deltanet :240-278) and the state copies of
  * deltanet_write_state (:208-238). Per value head h (key head
  * h / (n_v_heads / n_k_heads)), state S [head_dim][head_dim] (the second index
