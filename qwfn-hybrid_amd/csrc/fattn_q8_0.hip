@@ -146,8 +146,6 @@ struct fa_args {
     // a (batch, KV head, row group) on one XCD (they share its query rows)
     int32_t  pre_rgmap;
     uint32_t nbh_mul;      // ceil(2^32 / (B * nh_kv))
-    uint8_t * img;         // k_fa_pre's chunk images [KV head][chunk][IMG_BYTES], or null
-    int32_t  img_chunks;   // chunks of n_kv keys
     // fused append (app_n > 0): F32 rows [nh_kv * D] of K and V quantised into
     // cache rows app_row0 .. app_row0 + app_n - 1 before they are attended
     const char * app_k;
@@ -186,6 +184,8 @@ struct fa_args {
     unsigned long long * mctr;
     unsigned long long m_ebase;
     int32_t  m_nm;
+    uint8_t * img;         // k_fa_pre's chunk images [KV head][chunk][IMG_BYTES], or null
+    int32_t  img_chunks;   // chunks of n_kv keys
 };
 
 __device__ __forceinline__ uint32_t div_gqa(const fa_args & a, uint32_t r) {
@@ -4438,7 +4438,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
         for (int s = 0; s < SPW; s++) {
             const int slot = wave + PRE_WAVES * s;
             if (!dlive[s]) continue;
-            dma16_buf(slot >= ROW_SLOTS ? rm : IMG || slot < PRE_TDMA ? rk : rv, doff[s],
+            dma16_buf(IMG ? (slot < ROW_SLOTS ? rk : rm) : slot < PRE_TDMA ? rk : slot < ROW_SLOTS ? rv : rm, doff[s],
                       __builtin_amdgcn_readfirstlane(lds_addr(st + slot * 1024)));
         }
     };
@@ -4545,7 +4545,9 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
         __syncthreads();   // chunk c has landed; every wave is done with chunk c - 1 (and the prologue)
         if (c + 1 < n_chunks) issue_chunk(c + 1, stg + ((c + 1) & 1) * STAGE);
         if constexpr (!IMG) {
-            pre_convert<false>(st, vt, kq, skv, lane, wave);
+            int cl = lane;                 // opaque: the pass's addresses, hoisted, would spill
+            asm volatile("" : "+v"(cl));
+            pre_convert<false>(st, vt, kq, skv, cl, wave);
             __syncthreads();   // V^T and the scale tables of chunk c are complete
         }
 
