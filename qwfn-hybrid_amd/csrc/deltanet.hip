@@ -177,10 +177,11 @@ __global__ __launch_bounds__(DN_WAVES * 64) void k_gated_delta_net(dn_args a) {
 // lane. The decays enter as running products, never as quotients or
 // exponentials of differences, so that a decay of 0 (g = -inf) stays exact.
 //
-// A column whose d turns non-finite at token i (a non-finite input, or a state
-// that overflowed) is NaN from token i on in the recurrence; a product with the
-// zeros of the triangular matrices would carry that into earlier tokens, so
-// such a d enters the products as 0 and the column is set to NaN from i on.
+// A column whose d turns non-finite at token i (a non-finite input, a state that
+// overflowed, a d that overflows) is not finite from token i on in the
+// recurrence; a product with the zeros of the triangular matrices would carry
+// that into earlier tokens, so the right-hand sides and the solved d of such
+// tokens enter the products as 0 and the column is set to NaN from i on.
 //
 // What bounds it: the token-by-token kernel is a chain of T steps of 0.68 us (a
 // barrier and two cross-wave sums each); here a group of 64 tokens takes 8.6 us,
@@ -372,6 +373,22 @@ __device__ __forceinline__ void dc_invert(float * tinv, int m, int g) {
         if (4 * g + r >= H && m < H) tinv[(4 * g + r) * DC_MS + m] = -z[r];
 }
 
+// The first token of the lane's column whose x (tokens 4 g + r) is not finite, or `first` if that is
+// earlier; x is 0 from there on.
+__device__ __forceinline__ int dc_cut(f32x4 & x, int first, int g) {
+#pragma unroll
+    for (int r = 3; r >= 0; r--)
+        if (!__builtin_isfinite(x[r]) && 4 * g + r < first) first = 4 * g + r;
+    for (int o = 16; o < 64; o <<= 1) {
+        const int z = __shfl_xor(first, o);
+        first = z < first ? z : first;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if (4 * g + r >= first) x[r] = 0.f;
+    return first;
+}
+
 __global__ __launch_bounds__(DC_THREADS, 2) void k_gated_delta_chunks(dn_args a) {
     __shared__ dc_lds sm;
     // the blocks of a key head read the same k and q: consecutive heads on one XCD
@@ -453,26 +470,23 @@ __global__ __launch_bounds__(DC_THREADS, 2) void k_gated_delta_chunks(dn_args a)
 #pragma unroll
             for (int i = 0; i < DC_TILES; i++) Ot[2 * i + (r >> 1)] = mfma4(qx[i][r], S[i][r], Ot[2 * i + (r >> 1)]);
         const f32x4 M = (M0 + M1) + (M2 + M3);
-        f32x4 R;
-        bool bad = false;
+        f32x4 R, U = {};
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            R[r] = __fmaf_rn(-cc[r], M[r], v[r]) * bb[r];
-            bad |= !__builtin_isfinite(R[r]);
-        }
-        int first = DC_C;
-        if (__builtin_expect(__ballot(bad) != 0, 0)) {
-#pragma unroll
-            for (int r = 3; r >= 0; r--)
-                if (!__builtin_isfinite(R[r])) { first = 4 * g + r; R[r] = 0.f; }
-            for (int o = 16; o < 64; o <<= 1) {
-                const int z = __shfl_xor(first, o);
-                first = z < first ? z : first;
-            }
-        }
-        f32x4 U = {};
+        for (int r = 0; r < 4; r++) R[r] = __fmaf_rn(-cc[r], M[r], v[r]) * bb[r];
 #pragma unroll
         for (int r = 0; r < 4; r++) U = mfma4(tr[r], R[r], U);
+        // T_ii = 1, so a token whose R is not finite has no finite U either: one test for both
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= !__builtin_isfinite(U[r]);
+        int first = DC_C;
+        if (__builtin_expect(__ballot(bad) != 0, 0)) {
+            first = dc_cut(R, first, g);
+            U = f32x4{};
+#pragma unroll
+            for (int r = 0; r < 4; r++) U = mfma4(tr[r], R[r], U);
+            first = dc_cut(U, first, g);
+        }
         if (quarter == c) { Uf = U; ff = first; }
 #pragma unroll
         for (int i = 0; i < DC_TILES; i++) S[i] = S[i] * cend;

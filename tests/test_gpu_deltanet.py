@@ -174,3 +174,30 @@ def test_gated_delta_net_chunks_not_finite(gpu):
     badst[2:] = True
     assert not np.isfinite(st2[badst]).any()
     np.testing.assert_array_equal(st2[~badst], st[~badst])
+
+
+def test_gated_delta_net_chunks_overflow(gpu):
+    """Finite inputs whose d overflows at token 23 of a column (a value near the largest float at token 20, the key
+    of 23 opposite to 20's): that column is not finite from token 23 on, everything before it and every other column
+    is what it is without the overflow."""
+    T, nk, nv = 40, 1, 2
+    q, k, v, g, beta, s0 = _small(5, T, nk, nv)
+    g[:], beta[20:24] = 0.0, 1.0
+    k[23] = -k[20]
+    v[20, 1, 7] = 3.0e38
+    r_out, _ = _rule64(q, k, v, g, beta, s0)
+    v2 = v.copy()
+    v2[23, 1, 7] = 3.0e38                    # d = 3e38 - (-1) 3e38
+    say("gated_delta_net chunks with a d that overflows")
+    out, st, _ = _call(gpu, q, k, v2, g, beta, s0)
+    assert not np.isfinite(out[23:, 1, 7]).any() and not np.isfinite(st[1, :, 7]).any()
+    for sl in (slice(0, 20), slice(20, 23)):     # each at the scale of its own values
+        np.testing.assert_allclose(out[sl, 1, 7], r_out[sl, 1, 7], rtol=0, atol=1e-5 * np.abs(r_out[sl, 1, 7]).max())
+    v2[:, 1, 7] = 0.0
+    out0, st0, _ = _call(gpu, q, k, v2, g, beta, s0)
+    other = np.ones(out.shape, bool)
+    other[:, 1, 7] = False
+    np.testing.assert_array_equal(out[other], out0[other])
+    others = np.ones(st.shape, bool)
+    others[1, :, 7] = False
+    np.testing.assert_array_equal(st[others], st0[others])
