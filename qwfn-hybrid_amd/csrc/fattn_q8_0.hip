@@ -4545,9 +4545,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
         __syncthreads();   // chunk c has landed; every wave is done with chunk c - 1 (and the prologue)
         if (c + 1 < n_chunks) issue_chunk(c + 1, stg + ((c + 1) & 1) * STAGE);
         if constexpr (!IMG) {
-            int cl = lane;                 // opaque: the pass's addresses, hoisted, would spill
-            asm volatile("" : "+v"(cl));
-            pre_convert<false>(st, vt, kq, skv, cl, wave);
+            pre_convert<false>(st, vt, kq, skv, lane, wave);
             __syncthreads();   // V^T and the scale tables of chunk c are complete
         }
 
