@@ -4927,54 +4927,76 @@ int check_no_scratch() {
     return rc;
 }
 
-// Whether k_fa_pre's chunks are converted to images first: where a block walks
+// Whether k_fa_pre's chunks may be converted to images first: where a block walks
 // enough chunks to win the image launch back and enough row groups share a
 // chunk to win its bytes back. Attention op without and with images, 2 KV
 // heads: 33 chunks a block, 64 row groups 380 -> 328 us; 24 (48 x 2 row groups)
 // 272 -> 235; 11.5 (6) 167 -> 155; 9.5 (38) 142 -> 130; but 8.4 (16) 73.3 ->
-// 74.0; 6 (32) 58.1 -> 59.0; 2 (32) 34.8 -> 37.1.
-bool pre_images(int64_t B, int64_t n_rg, int64_t split_chunks) {
-    return B == 1 && n_rg >= 6 && split_chunks >= 9;
-}
+// 74.0; 6 (32) 58.1 -> 59.0; 2 (32) 34.8 -> 37.1. Above the line pre_cost
+// decides by what the image launch takes.
+bool pre_images(uint32_t n_rg, uint32_t split_chunks) { return n_rg >= 6 && split_chunks >= 9; }
 
-// The time of a k_fa_pre call of ns key splits in a block order (fa_args::
-// pre_rgmap), in us: an XCD's blocks run in rounds of its 32 CUs, each as long
-// as a block's chunks (5 us from images, else 6) and its prologue and epilogue
-// (6); the partials are written and read back, and the bytes the XCDs' L2s
-// cannot share (the f32 query rows once per split where units share an XCD, the
-// K/V rows once per XCD holding a KV head's row groups where splits do) come
-// again, at 4 TB/s. Measured where it decides (splits: us): 48 row groups, 72
+struct pre_shape {                // of a k_fa_pre call, for its planner
+    uint32_t nbh, n_rg, chunks;   // (batch, KV head) pairs, row groups, 64-key chunks
+    float    part, q_rep, kv_rep; // us of a split's partials, of the query rows once more, of K/V replicated
+    float    img;                 // us of the image launch
+};
+
+struct pre_choice { float cost; bool rgmap, images; };
+
+// The time of a k_fa_pre call of ns key splits, in us, with the better block
+// order (fa_args::pre_rgmap) and with images where they are cheaper: an XCD's
+// blocks run in rounds of its 32 CUs, each as long as a block's chunks (5 us
+// from images, else 6) and its prologue and epilogue (6); the image launch is
+// 5.5 us and its bytes (272 + 272 read, 800 written a key and KV head) at 6 TB/s;
+// the partials are written and read back, and the bytes the XCDs' L2s cannot
+// share (the f32 query rows once per split where units share an XCD, the K/V
+// rows once per XCD holding a KV head's row groups where splits do) come again,
+// at 4 TB/s. Measured where it decides (splits: us): 48 row groups, 72
 // chunks 3: 243, 4: 204, 5: 180, 6: 218, 8: 187; 38 row groups, 38 chunks 3: 93,
-// 4: 131; 19, 69 chunks 6: 88, 7: 117; 29, 133 chunks 4: 193, 5: 250.
+// 4: 131; 19, 69 chunks 6: 88, 7: 117; 29, 133 chunks 4: 193, 5: 250. Images
+// against none at one count: 16 row groups, 64 chunks, 7: 73.9, 75.2 (but 8,
+// without: 67.4); 7, 128 chunks, 15: 70.1, 69.6 (16: 63.6); 7, 1024 chunks, 16:
+// 339, 368, 36: 333, 356.
 // (32-bit and shifts: a call evaluates up to 256 split counts)
-float pre_cost(uint32_t nbh, uint32_t n_rg, uint32_t chunks, float part, float q_rep, float kv_rep, uint32_t ns, bool * rgmap) {
-    const uint32_t sc = (chunks + ns - 1) / ns;
-    const float block = (float) sc * (pre_images(1, n_rg, sc) ? 5.f : 6.f) + 6.f;
-    const uint32_t units = (nbh * ns + 7) >> 3, rgus = (nbh * n_rg + 7) >> 3;
-    const float c0 = (float) ((n_rg * units + 31) >> 5) * block + q_rep * (float) (ns - 1);
-    const float c1 = (float) ((ns * rgus + 31) >> 5) * block + kv_rep;
-    *rgmap = ns > 1 && c1 < c0;
-    return (*rgmap ? c1 : c0) + (ns > 1 ? part * (float) ns + 4.f : 0.f);
+pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
+    const uint32_t sc = (s.chunks + ns - 1) / ns;
+    const bool may = pre_images(s.n_rg, sc);
+    const uint32_t units = (s.nbh * ns + 7) >> 3, rgus = (s.nbh * s.n_rg + 7) >> 3;
+    const auto order = [&](uint32_t blocks, float again, bool rgmap) {
+        const float rounds = (float) ((blocks + 31) >> 5);
+        const float plain = rounds * ((float) sc * 6.f + 6.f), images = rounds * ((float) sc * 5.f + 6.f) + s.img;
+        return pre_choice{(may && images < plain ? images : plain) + again, rgmap, may && images < plain};
+    };
+    pre_choice c = order(s.n_rg * units, s.q_rep * (float) (ns - 1), false);
+    if (ns > 1) {
+        const pre_choice r = order(ns * rgus, s.kv_rep, true);
+        if (r.cost < c.cost) c = r;
+        c.cost += s.part * (float) ns + 4.f;
+    }
+    return c;
 }
 
-// k_fa_pre's key splits and block order: the cheapest count of whole chunks, at
-// least two a split, within three rounds of blocks (one where a call has few
-// row groups); forced: that count
-int64_t pre_splits(int64_t nbh, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced, bool * rgmap) {
-    const int64_t chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK), per = nbh * n_rg;
-    *rgmap = false;
+// k_fa_pre's key splits, block order and images: the cheapest count of whole
+// chunks, at least two a split, within three rounds of blocks (one where a call
+// has few row groups); forced: that count
+int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced,
+                   pre_choice * choice) {
+    const int64_t nbh = B * nh_kv, chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK), per = nbh * n_rg;
+    *choice = pre_choice{INFINITY, false, false};
     // (beyond 32 bits: more blocks than any split count is needed for)
     if (per >= (int64_t(1) << 24) || chunks >= (int64_t(1) << 24)) return forced ? std::min(forced, ns_cap) : 1;
-    const float part = 2.f * (float) (R * nbh) * D * 4 / 4e6f, q_rep = (float) R * D * 4 / 4e6f;
-    const float kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
+    pre_shape s{(uint32_t) nbh, (uint32_t) n_rg, (uint32_t) chunks, 0.f, 0.f, 0.f, 0.f};
+    s.part = 2.f * (float) (R * nbh) * D * 4 / 4e6f;
+    s.q_rep = (float) R * D * 4 / 4e6f;
+    s.kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
+    s.img = 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f;
     const int64_t most = std::min<int64_t>({(chunks + 1) / 2, ns_cap, std::max<int64_t>(1, (per < 8 ? 256 : 768) / per)});
     const int64_t lo = forced ? std::max<int64_t>(1, std::min(forced, ns_cap)) : 1, hi = forced ? lo : std::max<int64_t>(1, most);
     int64_t best = lo;
-    float cost = INFINITY;
     for (int64_t n = lo; n <= hi; n++) {
-        bool m;
-        const float c = pre_cost((uint32_t) nbh, (uint32_t) n_rg, (uint32_t) chunks, part, q_rep, kv_rep, (uint32_t) n, &m);
-        if (c < cost) { cost = c; best = n; *rgmap = m; }
+        const pre_choice c = pre_cost(s, (uint32_t) n);
+        if (c.cost < choice->cost) { *choice = c; best = n; }
     }
     return best;
 }
@@ -5082,8 +5104,8 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         pl->n_rg = (int32_t) ((R + PRE_ROWS - 1) / PRE_ROWS);
         pl->gqa = (int32_t) gqa;
         const int64_t chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK);
-        bool rgmap;
-        int64_t ns = pre_splits(B * nh_kv, pl->n_rg, R, n_kv, ns_cap, g_force_splits.load(std::memory_order_relaxed), &rgmap);
+        pre_choice choice;
+        int64_t ns = pre_splits(B, nh_kv, pl->n_rg, R, n_kv, ns_cap, g_force_splits.load(std::memory_order_relaxed), &choice);
         const int64_t split_len = (chunks + ns - 1) / ns * PRE_CK;
         ns = std::max<int64_t>(1, (n_kv + split_len - 1) / split_len);
         if (ns > MAX_SPLITS)
@@ -5093,13 +5115,13 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         pl->split_len = (int32_t) split_len;
         pl->max_span = split_len;
         pl->ragged = 0;
-        pl->pre_rgmap = ns > 1 && rgmap;
+        pl->pre_rgmap = ns > 1 && choice.rgmap;
         const size_t n_part = ns > 1 ? (size_t) (B * nh_kv * ns * R) : 0;
         size_t off = align256(n_part * D * sizeof(float));
         pl->off_ml = off;
         off = align256(off + n_part * sizeof(float2));
         pl->ws_base = pl->ws_bytes = std::max<size_t>(off, 256);
-        pl->img_chunks = pre_images(B, pl->n_rg, split_len / PRE_CK) ? (int32_t) chunks : 0;
+        pl->img_chunks = B == 1 && choice.images ? (int32_t) chunks : 0;
         if (pl->img_chunks) pl->ws_bytes += (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
         return QWFN_OK;
     }

@@ -1,0 +1,35 @@
+"""The planner of the prefill attention (key splits and chunk images), read off
+the workspace it asks for; no GPU."""
+import ctypes
+
+import pytest
+
+import qwfn_kv as K
+
+FAKE = 0x7F0000000000
+IMAGE = 51200        # bytes of a 64-key chunk's image, one KV head
+
+
+def workspace(T, nh, n_kv, B=1, nh_kv=2):
+    q = K.tensor(FAKE, K.TYPE_F32, (256, T, nh, B), (4, nh * 1024, 1024, T * nh * 1024))
+    k = K.tensor(FAKE, K.TYPE_Q8_0, (256, n_kv, nh_kv, B), (34, nh_kv * 272, 272, n_kv * nh_kv * 272))
+    r = ctypes.byref
+    return K.load().qwfn_fattn_workspace_size(r(q), r(k), r(k), None)
+
+
+def expected(T, nh, n_kv, B, splits, images, nh_kv=2):
+    up = lambda x: (x + 255) // 256 * 256
+    n = B * splits * T * nh                       # partial rows of all KV heads
+    base = up(up(n * 1024) + n * 8) if splits > 1 else 256
+    return base + (nh_kv * -(-n_kv // 64) * IMAGE if images else 0)
+
+
+# Attention op in us, the choice and what it was measured against: images that save less than their launch takes
+# (256 x 16 at 4096: 8 splits without 67.6, 7 with 73.8; 128 x 16 at 8192: 16 without 70.4, 15 with 74.5;
+# 100 x 16 at 8192: 16 without 66.8, 15 with 73.1), and images where they pay (512 x 16 at 16384: 321, without
+# 368; 512 x 24 at 4096: 5 splits 160, 3 202, without 237)
+@pytest.mark.parametrize("T,nh,n_kv,splits,images", [(256, 16, 4096, 8, False), (128, 16, 8192, 16, False),
+                                                     (100, 16, 8192, 16, False), (512, 16, 16384, 4, True),
+                                                     (512, 24, 4096, 5, True)])
+def test_prefill_plan(T, nh, n_kv, splits, images):
+    assert workspace(T, nh, n_kv) == expected(T, nh, n_kv, 1, splits, images)
