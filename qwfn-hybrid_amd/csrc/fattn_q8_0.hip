@@ -4939,7 +4939,7 @@ bool pre_images(uint32_t n_rg, uint32_t split_chunks) { return n_rg >= 6 && spli
 struct pre_shape {                // of a k_fa_pre call, for its planner
     uint32_t nbh, n_rg, chunks;   // (batch, KV head) pairs, row groups, 64-key chunks
     float    part, q_rep, kv_rep; // us of a split's partials, of the query rows once more, of K/V replicated
-    float    img;                 // us of the image launch
+    float    img;                 // us of the image launch; infinite where there can be none (batches)
 };
 
 struct pre_choice { float cost; bool rgmap, images; };
@@ -4990,7 +4990,7 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
     s.part = 2.f * (float) (R * nbh) * D * 4 / 4e6f;
     s.q_rep = (float) R * D * 4 / 4e6f;
     s.kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
-    s.img = 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f;
+    s.img = B == 1 ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;
     const int64_t most = std::min<int64_t>({(chunks + 1) / 2, ns_cap, std::max<int64_t>(1, (per < 8 ? 256 : 768) / per)});
     const int64_t lo = forced ? std::max<int64_t>(1, std::min(forced, ns_cap)) : 1, hi = forced ? lo : std::max<int64_t>(1, most);
     int64_t best = lo;
@@ -5121,7 +5121,7 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         pl->off_ml = off;
         off = align256(off + n_part * sizeof(float2));
         pl->ws_base = pl->ws_bytes = std::max<size_t>(off, 256);
-        pl->img_chunks = B == 1 && choice.images ? (int32_t) chunks : 0;
+        pl->img_chunks = choice.images ? (int32_t) chunks : 0;
         if (pl->img_chunks) pl->ws_bytes += (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
         return QWFN_OK;
     }
