@@ -162,9 +162,15 @@ int qwfn_kv_gather_segments_kv(const void * src_k, const void * src_v, size_t sr
  * least 256 bytes are asked for otherwise) and, for long query blocks over
  * many keys, the K/V rows converted once for all of them (800 bytes a key and
  * KV head, behind the partials: with a workspace that holds only the partials
- * the call converts them in every workgroup, slower, to the same bits); its
- * contents need not be preserved between calls. Calls that run at the same
- * time need distinct workspaces. */
+ * the call converts them in every workgroup, slower, to the same bits). The
+ * size is not monotone in T or n_kv. A prefill block (more than 32 query rows
+ * and at least 4 heads a KV head, a mask shared by the heads) takes fewer key
+ * splits where its workspace does not hold the partials of its own plan
+ * (slower, and other rounding), so a workspace sized for the longest block over
+ * the most keys serves the shorter ones too; the largest size over the shapes in
+ * use, the decode step among them, serves each best. Its contents need not be
+ * preserved between calls. Calls that run at the same time need distinct
+ * workspaces. */
 size_t qwfn_fattn_workspace_size(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,
                                  const qwfn_tensor * mask);
 int qwfn_flash_attn_ext_q8_0(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,

@@ -4939,7 +4939,7 @@ bool pre_images(uint32_t n_rg, uint32_t split_chunks) { return n_rg >= 6 && spli
 struct pre_shape {                // of a k_fa_pre call, for its planner
     uint32_t nbh, n_rg, chunks;   // (batch, KV head) pairs, row groups, 64-key chunks
     float    part, q_rep, kv_rep; // us of a split's partials, of the query rows once more, of K/V replicated
-    float    img;                 // us of the image launch; infinite where there can be none (batches)
+    float    img;                 // us of the image launch; infinite where there can be none
 };
 
 struct pre_choice { float cost; bool rgmap, images; };
@@ -4980,7 +4980,7 @@ pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
 // k_fa_pre's key splits, block order and images: the cheapest count of whole
 // chunks, at least two a split, within three rounds of blocks (one where a call
 // has few row groups); forced: that count
-int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced,
+int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced, bool images,
                    pre_choice * choice) {
     const int64_t nbh = B * nh_kv, chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK), per = nbh * n_rg;
     *choice = pre_choice{INFINITY, false, false};
@@ -4990,7 +4990,7 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
     s.part = 2.f * (float) (R * nbh) * D * 4 / 4e6f;
     s.q_rep = (float) R * D * 4 / 4e6f;
     s.kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
-    s.img = B == 1 ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;
+    s.img = B == 1 && images ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;
     const int64_t most = std::min<int64_t>({(chunks + 1) / 2, ns_cap, std::max<int64_t>(1, (per < 8 ? 256 : 768) / per)});
     const int64_t lo = forced ? std::max<int64_t>(1, std::min(forced, ns_cap)) : 1, hi = forced ? lo : std::max<int64_t>(1, most);
     int64_t best = lo;
@@ -5002,7 +5002,8 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
 }
 
 int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v, const qwfn_tensor * mask,
-               fa_plan * pl, const int64_t * seq_n_kv = nullptr, int64_t ns_cap = MAX_SPLITS, bool gather = false) {
+               fa_plan * pl, const int64_t * seq_n_kv = nullptr, int64_t ns_cap = MAX_SPLITS, bool gather = false,
+               bool images = true) {
     if (!q || !k || !v) return set_error(QWFN_EINVAL, "flash_attn_ext: NULL q/k/v");
     if (q->type != QWFN_TYPE_F32) return set_error(QWFN_EINVAL, "flash_attn_ext: q must be f32");
     if (k->type != QWFN_TYPE_Q8_0 || v->type != QWFN_TYPE_Q8_0)
@@ -5105,7 +5106,8 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         pl->gqa = (int32_t) gqa;
         const int64_t chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK);
         pre_choice choice;
-        int64_t ns = pre_splits(B, nh_kv, pl->n_rg, R, n_kv, ns_cap, g_force_splits.load(std::memory_order_relaxed), &choice);
+        int64_t ns = pre_splits(B, nh_kv, pl->n_rg, R, n_kv, ns_cap, g_force_splits.load(std::memory_order_relaxed),
+                                images, &choice);
         const int64_t split_len = (chunks + ns - 1) / ns * PRE_CK;
         ns = std::max<int64_t>(1, (n_kv + split_len - 1) / split_len);
         if (ns > MAX_SPLITS)
@@ -5397,12 +5399,17 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
     if (variant != QWFN_Q8_REF && variant != QWFN_Q8_X86) return set_error(QWFN_EINVAL, "flash_attn_ext: unknown variant");
     fa_plan pl{};
     if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, MAX_SPLITS, gat != nullptr)) return rc;
-    if (wsm == WS_SCRATCH && pl.ws_base > NOALLOC_SCRATCH_BYTES) {
-        // fewer key splits, so that their partials fit the scratch
+    // A room that does not hold the split partials of the plan: fewer key splits. For the library's scratch always;
+    // for a caller's workspace with k_fa_pre, whose split count goes by whole rounds of blocks and is not monotone
+    // in the keys or the query rows: one sized for a longer query block or more keys must do (a forced count asks
+    // for its own).
+    const size_t room = wsm == WS_SCRATCH ? NOALLOC_SCRATCH_BYTES : ws ? ws_bytes : SIZE_MAX;
+    const bool may_cap = wsm == WS_SCRATCH || (pl.kind == FA_PRE && room >= 256 && !g_force_splits.load(std::memory_order_relaxed));
+    if (pl.ws_base > room && may_cap) {
         const size_t per_split = (size_t) q->ne[3] * k->ne[2] * pl.R * (D * sizeof(float) + sizeof(float2));
-        const int64_t cap = std::max<int64_t>(1, (int64_t) ((NOALLOC_SCRATCH_BYTES - 512) / std::max<size_t>(per_split, 1)));
-        if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, cap, gat != nullptr)) return rc;
-        if (pl.ws_base > NOALLOC_SCRATCH_BYTES)
+        const int64_t cap = std::max<int64_t>(1, (int64_t) ((std::max<size_t>(room, 512) - 512) / std::max<size_t>(per_split, 1)));
+        if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, cap, gat != nullptr, false)) return rc;
+        if (wsm == WS_SCRATCH && pl.ws_base > room)
             return set_error(QWFN_ENOMEM, "flash_attn_ext_noalloc: the split partials need more than the 16 MiB scratch");
     }
     if (app)
@@ -5426,7 +5433,7 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
     }
     // no images where the workspace holds the partials only, or with rows that
     // the attention kernel itself appends
-    if (app || (wsm == WS_SCRATCH ? NOALLOC_SCRATCH_BYTES : ws ? ws_bytes : pl.ws_bytes) < pl.ws_bytes) {
+    if (app || room < pl.ws_bytes) {
         pl.img_chunks = 0;
         pl.ws_bytes = pl.ws_base;
     }
