@@ -4938,7 +4938,8 @@ bool pre_images(uint32_t n_rg, uint32_t split_chunks) { return n_rg >= 6 && spli
 
 struct pre_shape {                // of a k_fa_pre call, for its planner
     uint32_t nbh, n_rg, chunks;   // (batch, KV head) pairs, row groups, 64-key chunks
-    float    part, q_rep, kv_rep; // us of a split's partials, of the query rows once more, of K/V replicated
+    float    part;                // bytes of a split's partials
+    float    q_rep, kv_rep;       // us of the query rows once more, of K/V replicated
     float    img;                 // us of the image launch; infinite where there can be none
 };
 
@@ -4949,15 +4950,19 @@ struct pre_choice { float cost; bool rgmap, images; };
 // blocks run in rounds of its 32 CUs, each as long as a block's chunks (5 us
 // from images, else 6) and its prologue and epilogue (6); the image launch is
 // 5.5 us and its bytes (272 + 272 read, 800 written a key and KV head) at 6 TB/s;
-// the partials are written and read back, and the bytes the XCDs' L2s cannot
+// the partials are written and read back, at 10 TB/s what the L2s hold (32 MB),
+// at 4 what they do not, and merged (4; 12 above MERGE_ROWS_SPLITS, by
+// k_fattn_merge, which reads the dead ones too); the bytes the XCDs' L2s cannot
 // share (the f32 query rows once per split where units share an XCD, the K/V
 // rows once per XCD holding a KV head's row groups where splits do) come again,
-// at 4 TB/s. Measured where it decides (splits: us): 48 row groups, 72
-// chunks 3: 243, 4: 204, 5: 180, 6: 218, 8: 187; 38 row groups, 38 chunks 3: 93,
-// 4: 131; 19, 69 chunks 6: 88, 7: 117; 29, 133 chunks 4: 193, 5: 250. Images
-// against none at one count: 16 row groups, 64 chunks, 7: 73.9, 75.2 (but 8,
-// without: 67.4); 7, 128 chunks, 15: 70.1, 69.6 (16: 63.6); 7, 1024 chunks, 16:
-// 339, 368, 36: 333, 356.
+// at 4 TB/s. Measured where it decides (splits: us): 48 row groups, 72 chunks
+// 3: 243, 4: 204, 5: 180, 6: 218, 8: 187; 38 row groups, 38 chunks 3: 93, 4: 131;
+// 19, 69 chunks 6: 88, 7: 117; 29, 133 chunks 4: 193, 5: 250. Images against none
+// at one count: 16 row groups, 64 chunks, 7: 73.9, 75.2 (but 8, without: 67.4);
+// 7, 128 chunks, 15: 70.1, 69.6 (16: 63.6); 7, 1024 chunks, 16: 339, 368, 36: 333,
+// 356. Few keys, 80 row groups, 4 chunks 1: 39.8, 2: 29.6; 24, 9 chunks 3: 38.6,
+// 5: 34.3. Across 16 splits: 12 row groups, 128 chunks 16: 64.2, 19: 69.2; 24,
+// 1024 chunks 10: 516, 32: 541.
 // (32-bit and shifts: a call evaluates up to 256 split counts)
 pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
     const uint32_t sc = (s.chunks + ns - 1) / ns;
@@ -4972,7 +4977,8 @@ pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
     if (ns > 1) {
         const pre_choice r = order(ns * rgus, s.kv_rep, true);
         if (r.cost < c.cost) c = r;
-        c.cost += s.part * (float) ns + 4.f;
+        const float bytes = s.part * (float) ns, l2 = std::min(bytes, 32e6f);
+        c.cost += 2.f * (l2 / 10e6f + (bytes - l2) / 4e6f) + (ns > MERGE_ROWS_SPLITS ? 12.f : 4.f);
     }
     return c;
 }
@@ -4987,7 +4993,7 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
     // (beyond 32 bits: more blocks than any split count is needed for)
     if (per >= (int64_t(1) << 24) || chunks >= (int64_t(1) << 24)) return forced ? std::min(forced, ns_cap) : 1;
     pre_shape s{(uint32_t) nbh, (uint32_t) n_rg, (uint32_t) chunks, 0.f, 0.f, 0.f, 0.f};
-    s.part = 2.f * (float) (R * nbh) * D * 4 / 4e6f;
+    s.part = (float) (R * nbh) * (D + 2) * 4;
     s.q_rep = (float) R * D * 4 / 4e6f;
     s.kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
     s.img = B == 1 && images ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;

@@ -40,3 +40,14 @@ def test_prefill_plan(T, nh, n_kv, splits, images):
 @pytest.mark.parametrize("T,nh,n_kv,B,splits", [(128, 16, 4096, 2, 8), (512, 24, 2048, 2, 4), (200, 24, 4096, 4, 5)])
 def test_prefill_plan_batch(T, nh, n_kv, B, splits):
     assert workspace(T, nh, n_kv, B) == expected(T, nh, n_kv, B, splits, False)
+
+
+# What the splits' partials cost (before and after, us): cheap while the L2s hold them (256 x 32 at 256 keys on 8 KV
+# heads: one split 39.8, two 28.9; 256 x 16 at 256, 2 sequences: 40.4, 28.8; 256 x 24 at 513: 3 splits 38.6, 5 34.3),
+# dear beyond 16 splits, where the other merge reads them (64 x 24 at 8192 on 4 KV heads: 19 splits 69.3, 16 67.1;
+# 128 x 24 at 65536: 32 splits 541, 10 516)
+@pytest.mark.parametrize("T,nh,n_kv,B,nh_kv,splits,images", [(256, 32, 256, 1, 8, 2, False), (256, 16, 256, 2, 2, 2, False),
+                                                             (256, 24, 513, 1, 2, 5, False), (64, 24, 8192, 1, 4, 16, False),
+                                                             (128, 24, 65536, 1, 2, 10, True)])
+def test_prefill_plan_partials(T, nh, n_kv, B, nh_kv, splits, images):
+    assert workspace(T, nh, n_kv, B, nh_kv) == expected(T, nh, n_kv, B, splits, images, nh_kv)
