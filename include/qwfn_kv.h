@@ -161,16 +161,15 @@ int qwfn_kv_gather_segments_kv(const void * src_k, const void * src_v, size_t sr
  * holds the split partials when the keys are split across workgroups (at
  * least 256 bytes are asked for otherwise) and, for long query blocks over
  * many keys, the K/V rows converted once for all of them (800 bytes a key and
- * KV head, behind the partials: with a workspace that holds only the partials
- * the call converts them in every workgroup, slower, to the same bits). The
- * size is not monotone in T or n_kv. A prefill block (more than 32 query rows
- * and at least 4 heads a KV head, a mask shared by the heads) takes fewer key
- * splits where its workspace does not hold the partials of its own plan
- * (slower, and other rounding), so a workspace sized for the longest block over
- * the most keys serves the shorter ones too; the largest size over the shapes in
- * use, the decode step among them, serves each best. Its contents need not be
- * preserved between calls. Calls that run at the same time need distinct
- * workspaces. */
+ * KV head, behind the partials). The size is not monotone in T or n_kv, but a
+ * prefill block (more than 32 query rows and at least 4 heads a KV head, a mask
+ * shared by the heads) is planned within the workspace it is given: with less
+ * than its size it takes fewer key splits, or converts in every workgroup, or
+ * both, whichever is faster (slower than with all of it, and other rounding).
+ * So a workspace sized for the longest block over the most keys serves the
+ * shorter ones too; the largest size over the shapes in use, the decode step
+ * among them, serves each best. Its contents need not be preserved between
+ * calls. Calls that run at the same time need distinct workspaces. */
 size_t qwfn_fattn_workspace_size(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,
                                  const qwfn_tensor * mask);
 int qwfn_flash_attn_ext_q8_0(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,
@@ -180,10 +179,11 @@ int qwfn_flash_attn_ext_q8_0(const qwfn_tensor * q, const qwfn_tensor * k, const
 /* qwfn_flash_attn_ext_q8_0 without a workspace argument and without any
  * device allocation: no counterpart in the reference; for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc). The split partials go to a 16 MiB scratch array inside the
- * library's code object (one per GPU, held until the process ends); when a
- * call's partials would not fit, it uses fewer key splits (the result then
- * differs from qwfn_flash_attn_ext_q8_0's only by float rounding). Every call on
+ * forbid hipMalloc). What would lie in the workspace goes to a 16 MiB scratch
+ * array inside the library's code object (one per GPU, held until the process
+ * ends); when a call's workspace size is more, it is planned within the 16 MiB
+ * (the result then differs from qwfn_flash_attn_ext_q8_0's only by float
+ * rounding). Every call on
  * a GPU shares that GPU's scratch: calls that overlap on one GPU (two streams,
  * or two threads) race and give wrong results. */
 int qwfn_flash_attn_ext_q8_0_noalloc(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v,

@@ -4940,7 +4940,7 @@ struct pre_shape {                // of a k_fa_pre call, for its planner
     uint32_t nbh, n_rg, chunks;   // (batch, KV head) pairs, row groups, 64-key chunks
     float    part;                // bytes of a split's partials
     float    q_rep, kv_rep;       // us of the query rows once more, of K/V replicated
-    float    img;                 // us of the image launch; infinite where there can be none
+    float    img;                 // us of the image launch; infinite where there can be none (batches, no room)
 };
 
 struct pre_choice { float cost; bool rgmap, images; };
@@ -4983,10 +4983,18 @@ pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
     return c;
 }
 
+// Workspace bytes of the partials of ns key splits: O rows, then (max, sum) pairs at *off_ml
+size_t part_bytes(int64_t nbh, int64_t ns, int64_t R, size_t * off_ml = nullptr) {
+    const size_t n = ns > 1 ? (size_t) (nbh * ns * R) : 0, o = align256(n * D * sizeof(float));
+    if (off_ml) *off_ml = o;
+    return std::max<size_t>(align256(o + n * sizeof(float2)), 256);
+}
+
 // k_fa_pre's key splits, block order and images: the cheapest count of whole
 // chunks, at least two a split, within three rounds of blocks (one where a call
-// has few row groups); forced: that count
-int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced, bool images,
+// has few row groups), whose partials `room` bytes hold, with images where it
+// holds them too; forced: that count
+int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_kv, int64_t ns_cap, int64_t forced, size_t room,
                    pre_choice * choice) {
     const int64_t nbh = B * nh_kv, chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK), per = nbh * n_rg;
     *choice = pre_choice{INFINITY, false, false};
@@ -4996,11 +5004,16 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
     s.part = (float) (R * nbh) * (D + 2) * 4;
     s.q_rep = (float) R * D * 4 / 4e6f;
     s.kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
-    s.img = B == 1 && images ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;
+    const float img = B == 1 ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;
     const int64_t most = std::min<int64_t>({(chunks + 1) / 2, ns_cap, std::max<int64_t>(1, (per < 8 ? 256 : 768) / per)});
     const int64_t lo = forced ? std::max<int64_t>(1, std::min(forced, ns_cap)) : 1, hi = forced ? lo : std::max<int64_t>(1, most);
     int64_t best = lo;
+    const size_t img_bytes = (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
     for (int64_t n = lo; n <= hi; n++) {
+        const int64_t sc = (chunks + n - 1) / n;
+        const size_t bytes = part_bytes(nbh, (chunks + sc - 1) / sc, R);
+        if (bytes > room && !forced) continue;
+        s.img = bytes <= room && room - bytes >= img_bytes ? img : INFINITY;
         const pre_choice c = pre_cost(s, (uint32_t) n);
         if (c.cost < choice->cost) { *choice = c; best = n; }
     }
@@ -5009,7 +5022,7 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
 
 int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * v, const qwfn_tensor * mask,
                fa_plan * pl, const int64_t * seq_n_kv = nullptr, int64_t ns_cap = MAX_SPLITS, bool gather = false,
-               bool images = true) {
+               size_t room = SIZE_MAX) {
     if (!q || !k || !v) return set_error(QWFN_EINVAL, "flash_attn_ext: NULL q/k/v");
     if (q->type != QWFN_TYPE_F32) return set_error(QWFN_EINVAL, "flash_attn_ext: q must be f32");
     if (k->type != QWFN_TYPE_Q8_0 || v->type != QWFN_TYPE_Q8_0)
@@ -5113,7 +5126,7 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         const int64_t chunks = std::max<int64_t>(1, (n_kv + PRE_CK - 1) / PRE_CK);
         pre_choice choice;
         int64_t ns = pre_splits(B, nh_kv, pl->n_rg, R, n_kv, ns_cap, g_force_splits.load(std::memory_order_relaxed),
-                                images, &choice);
+                                room, &choice);
         const int64_t split_len = (chunks + ns - 1) / ns * PRE_CK;
         ns = std::max<int64_t>(1, (n_kv + split_len - 1) / split_len);
         if (ns > MAX_SPLITS)
@@ -5124,11 +5137,7 @@ int plan_fattn(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor *
         pl->max_span = split_len;
         pl->ragged = 0;
         pl->pre_rgmap = ns > 1 && choice.rgmap;
-        const size_t n_part = ns > 1 ? (size_t) (B * nh_kv * ns * R) : 0;
-        size_t off = align256(n_part * D * sizeof(float));
-        pl->off_ml = off;
-        off = align256(off + n_part * sizeof(float2));
-        pl->ws_base = pl->ws_bytes = std::max<size_t>(off, 256);
+        pl->ws_base = pl->ws_bytes = part_bytes(B * nh_kv, ns, R, &pl->off_ml);
         pl->img_chunks = choice.images ? (int32_t) chunks : 0;
         if (pl->img_chunks) pl->ws_bytes += (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
         return QWFN_OK;
@@ -5404,18 +5413,16 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
     if (!(std::isfinite(scale))) return set_error(QWFN_EINVAL, "flash_attn_ext: scale must be finite");
     if (variant != QWFN_Q8_REF && variant != QWFN_Q8_X86) return set_error(QWFN_EINVAL, "flash_attn_ext: unknown variant");
     fa_plan pl{};
-    if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, MAX_SPLITS, gat != nullptr)) return rc;
-    // A room that does not hold the split partials of the plan: fewer key splits. For the library's scratch always;
-    // for a caller's workspace with k_fa_pre, whose split count goes by whole rounds of blocks and is not monotone
-    // in the keys or the query rows: one sized for a longer query block or more keys must do (a forced count asks
-    // for its own).
+    // k_fa_pre plans within the room there is: its split count goes by whole rounds of blocks and is not monotone in
+    // the keys or the query rows, so a workspace sized for a longer query block or more keys must do
     const size_t room = wsm == WS_SCRATCH ? NOALLOC_SCRATCH_BYTES : ws ? ws_bytes : SIZE_MAX;
-    const bool may_cap = wsm == WS_SCRATCH || (pl.kind == FA_PRE && room >= 256 && !g_force_splits.load(std::memory_order_relaxed));
-    if (pl.ws_base > room && may_cap) {
+    if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, MAX_SPLITS, gat != nullptr, room)) return rc;
+    if (wsm == WS_SCRATCH && pl.ws_base > room) {
+        // fewer key splits, so that their partials fit the scratch
         const size_t per_split = (size_t) q->ne[3] * k->ne[2] * pl.R * (D * sizeof(float) + sizeof(float2));
-        const int64_t cap = std::max<int64_t>(1, (int64_t) ((std::max<size_t>(room, 512) - 512) / std::max<size_t>(per_split, 1)));
-        if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, cap, gat != nullptr, false)) return rc;
-        if (wsm == WS_SCRATCH && pl.ws_base > room)
+        const int64_t cap = std::max<int64_t>(1, (int64_t) ((room - 512) / std::max<size_t>(per_split, 1)));
+        if (int rc = plan_fattn(q, k, v, mask, &pl, seq_n_kv, cap, gat != nullptr, room)) return rc;
+        if (pl.ws_base > room)
             return set_error(QWFN_ENOMEM, "flash_attn_ext_noalloc: the split partials need more than the 16 MiB scratch");
     }
     if (app)
@@ -5437,8 +5444,8 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
                            dim3(256), 0, as_stream(stream), (float *) dst->data, n);
         return hip_check(hipGetLastError(), "flash_attn zero fill");
     }
-    // no images where the workspace holds the partials only, or with rows that
-    // the attention kernel itself appends
+    // no images where the room holds a forced count's partials only, or with rows that the attention kernel itself
+    // appends (planned as the call without them, so that its result is the same bits)
     if (app || room < pl.ws_bytes) {
         pl.img_chunks = 0;
         pl.ws_bytes = pl.ws_base;
