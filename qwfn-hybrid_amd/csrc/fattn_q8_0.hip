@@ -5455,8 +5455,14 @@ int fattn_run(const qwfn_tensor * q, const qwfn_tensor * k, const qwfn_tensor * 
     } else if (ws) {
         if (ws_bytes < pl.ws_bytes) return set_error(QWFN_ENOMEM, "flash_attn_ext: workspace too small");
         if (!is_aligned(ws, 256)) return set_error(QWFN_EALIGN, "flash_attn_ext: workspace must be 256-byte aligned");
-    } else if (int rc = library_workspace(pl.ws_bytes, as_stream(stream), &ws)) {
-        return rc;
+    } else {
+        size_t got = 0;
+        if (int rc = library_workspace(pl.ws_bytes, pl.ws_base, as_stream(stream), &ws, &got)) return rc;
+        if (got < pl.ws_bytes) {
+            // the device had room for the partials only
+            pl.img_chunks = 0;
+            pl.ws_bytes = pl.ws_base;
+        }
     }
     if (int rc = check_no_scratch()) return rc;
 

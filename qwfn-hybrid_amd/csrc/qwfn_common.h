@@ -47,10 +47,11 @@ int  set_error2(int code, const char * what, const char * msg) noexcept;
 int  hip_check(hipError_t e, const char * what) noexcept;
 // Per-device status word (uint32 flags); created by qwfn_init or on first use.
 int  status_word(uint32_t ** out);
-// Library-owned workspace of at least `bytes` on the current device, shared by
+// Library-owned workspace of at least `bytes` on the current device, or where the
+// device has no such memory of at least `least`; *got: its size. Shared by
 // every call on that device that passes no workspace. Refused while `stream`
 // is being captured into a graph (a later, larger call frees the buffer).
-int  library_workspace(size_t bytes, hipStream_t stream, void ** out);
+int  library_workspace(size_t bytes, size_t least, hipStream_t stream, void ** out, size_t * got);
 
 // The body of an extern "C" entry point: no C++ exception crosses the ABI. A
 // host allocation failure returns QWFN_ENOMEM (as the reference's

@@ -1,6 +1,7 @@
 // Error strings, per-device status word and library-owned workspace.
 #include "qwfn_common.h"
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 
@@ -16,6 +17,7 @@ struct device_slot {
     uint32_t * status = nullptr;   // device word: DEVERR_* bits
     void *     ws     = nullptr;   // library-owned attention workspace
     size_t     ws_bytes = 0;
+    size_t     ws_refused = SIZE_MAX;   // the smallest size the device could not give; cleared when it gives as much
 };
 // One slot per device index, at a fixed address for the life of the process
 // (a pointer to a slot stays valid whatever other threads do).
@@ -74,7 +76,7 @@ int status_word(uint32_t ** out) {
     return QWFN_OK;
 }
 
-int library_workspace(size_t bytes, hipStream_t stream, void ** out) {
+int library_workspace(size_t bytes, size_t least, hipStream_t stream, void ** out, size_t * got) {
     // The buffer is allocated (and regrown) by the library, so its address must
     // never be recorded into a graph: a later, larger call frees it.
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -84,7 +86,10 @@ int library_workspace(size_t bytes, hipStream_t stream, void ** out) {
     device_slot * s = nullptr;
     if (int rc = current_slot(&s)) return rc;
     std::lock_guard<std::mutex> lk(g_mu);
-    if (s->ws_bytes < bytes) {
+    // a size that was refused is not asked for again at every call (each time freeing the buffer and waiting)
+    const size_t need = bytes < s->ws_refused ? bytes : least;
+    if (s->ws_bytes < need) {
+        const size_t old = s->ws_bytes;
         if (s->ws) {
             // work already queued on any stream may still use the old buffer
             QWFN_HIP_TRY(hipDeviceSynchronize());
@@ -92,11 +97,29 @@ int library_workspace(size_t bytes, hipStream_t stream, void ** out) {
             s->ws = nullptr;
             s->ws_bytes = 0;
         }
-        size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
-        QWFN_HIP_TRY(hipMalloc(&s->ws, want));
-        s->ws_bytes = want;
+        // Grown by half at least: a context that grows call by call asks for a little more each time. Where the
+        // device cannot give that, what the call needs, then what there was or the least it can run with.
+        const size_t sizes[4] = {std::max({need, old + old / 2, size_t(1) << 20}), need, std::max(old, least), least};
+        int rc = QWFN_OK;
+        for (int i = 0; i < 4 && !s->ws; i++) {
+            if (i > 0 && sizes[i] >= sizes[i - 1]) continue;
+            void * p = nullptr;
+            rc = hip_check(hipMalloc(&p, sizes[i]), "workspace");
+            if (rc == QWFN_OK) {
+                s->ws = p;
+                s->ws_bytes = sizes[i];
+                if (sizes[i] >= s->ws_refused) s->ws_refused = SIZE_MAX;
+            } else if (rc == QWFN_ENOMEM) {
+                (void) hipGetLastError();   // else the next launch's check reports it
+                if (sizes[i] <= need) s->ws_refused = std::min(s->ws_refused, sizes[i]);
+            } else {
+                break;
+            }
+        }
+        if (!s->ws) return rc;
     }
     *out = s->ws;
+    *got = s->ws_bytes;
     return QWFN_OK;
 }
 

@@ -12,6 +12,10 @@
 // returns false on std::bad_alloc, qwfn_engine.cpp:1022-1025), and that a
 // pool save that fails on a host allocation leaves the pool exactly as it was
 // (device errors after the last allocation are outside what this checks).
+//
+// The device allocations behind the library's own attention workspace are
+// played by a device of a few megabytes below (the HIP calls that it makes are
+// defined here), to check how it grows and what it does when there is no room.
 #include "qwfn_kv.h"
 #include "qwfn_state.h"
 
@@ -255,11 +259,73 @@ static void check_validation() {
     CHECK(qwfn_qsa_bucket(100, 0, 10) == 0);
 }
 
+// ------------------------------------------------ the library's workspace
+
+// A device with g_room bytes, or none (any call fails, as without a GPU)
+static bool   g_device = false;
+static size_t g_room = 0, g_used = 0, g_last_size = 0;
+static int    g_mallocs = 0, g_syncs = 0, g_last_hip = 0;
+static int hip_result(int e) { return e ? g_last_hip = e : 0; }
+struct ihipStream_t;
+extern "C" {
+int hipMalloc(void ** p, size_t n) {
+    if (!g_device) return hip_result(100);   // hipErrorNoDevice
+    g_mallocs++;
+    if (g_used + n > g_room) return hip_result(2);   // hipErrorOutOfMemory
+    g_used += g_last_size = n;
+    *p = (void *) 0x7F0000000000;
+    return 0;
+}
+int hipFree(void *) {
+    if (!g_device) return hip_result(100);
+    g_used -= g_last_size;   // one buffer at a time
+    return 0;
+}
+int hipDeviceSynchronize() { g_syncs++; return hip_result(g_device ? 0 : 100); }
+int hipGetDevice(int * d) { *d = 0; return hip_result(g_device ? 0 : 100); }
+int hipStreamIsCapturing(ihipStream_t *, int * status) { *status = 0; return hip_result(g_device ? 0 : 100); }
+int hipGetLastError() { const int e = g_last_hip; g_last_hip = 0; return e; }
+}
+namespace qwfn {
+int library_workspace(size_t bytes, size_t least, ihipStream_t * stream, void ** out, size_t * got);
+}
+
+static void check_library_workspace() {
+    constexpr size_t MB = size_t(1) << 20;
+    void * p = nullptr;
+    size_t got = 0;
+    auto call = [&](size_t bytes, size_t least) { got = 0; return qwfn::library_workspace(bytes, least, nullptr, &p, &got); };
+    g_device = true;
+    g_room = 100 * MB;
+    CHECK(call(1000, 1000) == QWFN_OK && got == MB && g_syncs == 0);
+    // a context that grows by 1 MB a call, 20 to 60 MB: the buffer is regrown a few times only
+    int before = g_mallocs;
+    for (size_t n = 20; n <= 60; n++) CHECK(call(n * MB, 8 * MB) == QWFN_OK && got >= n * MB && got <= 90 * MB);
+    CHECK(g_mallocs - before <= 5 && g_syncs <= 5);
+    // no room for half as much again: exactly what is asked for
+    CHECK(call(99 * MB, 8 * MB) == QWFN_OK && got == 99 * MB && g_last_hip == 0);
+    // no room for that either: the least, no error left behind, and no further tries while it is known
+    CHECK(call(101 * MB, 40 * MB) == QWFN_OK && got == 99 * MB);
+    g_room = 50 * MB;   // another allocation has taken the rest
+    CHECK(call(200 * MB, 100 * MB) == QWFN_ENOMEM && g_last_hip == 0);
+    CHECK(call(80 * MB, 40 * MB) == QWFN_OK && got >= 40 * MB && got <= 50 * MB && g_last_hip == 0);
+    before = g_mallocs;
+    const int syncs = g_syncs;
+    for (int i = 0; i < 3; i++) CHECK(call(80 * MB, 40 * MB) == QWFN_OK && got < 80 * MB);
+    CHECK(g_mallocs == before && g_syncs == syncs);
+    // what is needed at least is always asked for, and once it is given the larger sizes are tried again
+    g_room = 300 * MB;
+    CHECK(call(120 * MB, 90 * MB) == QWFN_OK && got >= 90 * MB);
+    CHECK(call(120 * MB, 90 * MB) == QWFN_OK && got >= 120 * MB);
+    g_device = false;
+}
+
 int main() {
     check_state_layout();
     check_pool();
     check_oom_paths();
     check_validation();
+    check_library_workspace();
     if (g_fail) {
         std::fprintf(stderr, "%d host checks failed\n", g_fail);
         return 1;
