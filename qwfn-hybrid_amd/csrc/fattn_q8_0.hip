@@ -4132,7 +4132,7 @@ __global__ __launch_bounds__(VS_WAVES * 64, 2) void k_fa_vs(fa_args a) {
 // arithmetic. A wave whose rows see none of the
 // chunk's keys (a causal mask's upper triangle) skips it.
 //
-// Where many row groups walk the same chunks (pre_images), the conversion is
+// Where many row groups walk the same chunks (pre_cost), the conversion is
 // done once: k_fa_pre_image writes every chunk as k_fa_pre reads it from LDS
 // into the call's workspace, and the key loop is DMAs, one barrier a chunk and
 // the arithmetic. The conversion and its barrier were 1.4 us of a chunk's 6.1;
@@ -4311,8 +4311,8 @@ __device__ __forceinline__ void pre_convert(const uint8_t * st, uint8_t * vt, ui
 
 // The images of chunk blockIdx.x of KV head blockIdx.y: the rows to LDS, the
 // conversion over them, the image out. Keys past n_kv are zeros (k_fa_pre masks
-// them). Bound by its bytes (272 + 272 in, 800 out a key and head): 18 us of a
-// profiled launch at 16896 keys and 2 heads, 45 MB.
+// them). Bound by its bytes (272 + 272 in, 800 out a key and head): 10.3 us at
+// 16896 keys and 2 heads, 45 MB.
 __global__ __launch_bounds__(PRE_WAVES * 64) void k_fa_pre_image(fa_args a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[IMG_BYTES];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -4927,14 +4927,14 @@ int check_no_scratch() {
     return rc;
 }
 
-// Whether k_fa_pre's chunks may be converted to images first: where a block walks
+// k_fa_pre's chunks may be converted to images first where a block walks
 // enough chunks to win the image launch back and enough row groups share a
 // chunk to win its bytes back. Attention op without and with images, 2 KV
 // heads: 33 chunks a block, 64 row groups 380 -> 328 us; 24 (48 x 2 row groups)
 // 272 -> 235; 11.5 (6) 167 -> 155; 9.5 (38) 142 -> 130; but 8.4 (16) 73.3 ->
 // 74.0; 6 (32) 58.1 -> 59.0; 2 (32) 34.8 -> 37.1. Above the line pre_cost
 // decides by what the image launch takes.
-bool pre_images(uint32_t n_rg, uint32_t split_chunks) { return n_rg >= 6 && split_chunks >= 9; }
+constexpr uint32_t PRE_IMG_RG = 6, PRE_IMG_CHUNKS = 9;
 
 struct pre_shape {                // of a k_fa_pre call, for its planner
     uint32_t nbh, n_rg, chunks;   // (batch, KV head) pairs, row groups, 64-key chunks
@@ -4963,10 +4963,9 @@ struct pre_choice { float cost; bool rgmap, images; };
 // 356. Few keys, 80 row groups, 4 chunks 1: 39.8, 2: 29.6; 24, 9 chunks 3: 38.6,
 // 5: 34.3. Across 16 splits: 12 row groups, 128 chunks 16: 64.2, 19: 69.2; 24,
 // 1024 chunks 10: 516, 32: 541.
-// (32-bit and shifts: a call evaluates up to 256 split counts)
-pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
-    const uint32_t sc = (s.chunks + ns - 1) / ns;
-    const bool may = pre_images(s.n_rg, sc);
+// (32-bit and shifts: a call evaluates every split length of up to 256 counts)
+inline pre_choice pre_cost(const pre_shape & s, uint32_t ns, uint32_t sc) {   // sc: chunks of a split
+    const bool may = s.n_rg >= PRE_IMG_RG && sc >= PRE_IMG_CHUNKS;
     const uint32_t units = (s.nbh * ns + 7) >> 3, rgus = (s.nbh * s.n_rg + 7) >> 3;
     const auto order = [&](uint32_t blocks, float again, bool rgmap) {
         const float rounds = (float) ((blocks + 31) >> 5);
@@ -4978,7 +4977,7 @@ pre_choice pre_cost(const pre_shape & s, uint32_t ns) {
         const pre_choice r = order(ns * rgus, s.kv_rep, true);
         if (r.cost < c.cost) c = r;
         const float bytes = s.part * (float) ns, l2 = std::min(bytes, 32e6f);
-        c.cost += 2.f * (l2 / 10e6f + (bytes - l2) / 4e6f) + (ns > MERGE_ROWS_SPLITS ? 12.f : 4.f);
+        c.cost += l2 * (2.f / 10e6f) + (bytes - l2) * (2.f / 4e6f) + (ns > MERGE_ROWS_SPLITS ? 12.f : 4.f);
     }
     return c;
 }
@@ -5001,20 +5000,33 @@ int64_t pre_splits(int64_t B, int64_t nh_kv, int64_t n_rg, int64_t R, int64_t n_
     // (beyond 32 bits: more blocks than any split count is needed for)
     if (per >= (int64_t(1) << 24) || chunks >= (int64_t(1) << 24)) return forced ? std::min(forced, ns_cap) : 1;
     pre_shape s{(uint32_t) nbh, (uint32_t) n_rg, (uint32_t) chunks, 0.f, 0.f, 0.f, 0.f};
-    s.part = (float) (R * nbh) * (D + 2) * 4;
+    const size_t split_bytes = (size_t) (R * nbh) * (D * sizeof(float) + sizeof(float2));
+    s.part = (float) split_bytes;
     s.q_rep = (float) R * D * 4 / 4e6f;
     s.kv_rep = (float) n_kv * (2 * NBLK * QBLOCK) * (float) (std::max<int64_t>(1, 8 / nbh) - 1) / 4e6f;
-    const float img = B == 1 ? 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f : INFINITY;
     const int64_t most = std::min<int64_t>({(chunks + 1) / 2, ns_cap, std::max<int64_t>(1, (per < 8 ? 256 : 768) / per)});
     const int64_t lo = forced ? std::max<int64_t>(1, std::min(forced, ns_cap)) : 1, hi = forced ? lo : std::max<int64_t>(1, most);
+    // the largest count of at most hi whose partials r bytes hold
+    const auto fits = [&](size_t r) {
+        if (r < 256) return int64_t(0);
+        int64_t n = std::max<int64_t>(1, (int64_t) std::min<size_t>((size_t) hi, r / split_bytes));
+        while (n > 1 && part_bytes(nbh, n, R) > r) n--;
+        return n;
+    };
+    const int64_t sc_lo = (chunks + lo - 1) / lo;
+    const size_t img_bytes = (size_t) nh_kv * (size_t) chunks * IMG_BYTES, img_room = room > img_bytes ? room - img_bytes : 0;
+    const int64_t n_max = forced ? hi : fits(room);
+    const int64_t n_img = B > 1 || n_rg < PRE_IMG_RG ? 0 : !forced ? fits(img_room)
+                        : part_bytes(nbh, (chunks + sc_lo - 1) / sc_lo, R) <= img_room ? hi : 0;
+    const float img = 5.5f + (float) (n_kv * nh_kv) * (2 * NBLK * QBLOCK + IMG_BYTES / PRE_CK) / 6e6f;
     int64_t best = lo;
-    const size_t img_bytes = (size_t) nh_kv * (size_t) chunks * IMG_BYTES;
-    for (int64_t n = lo; n <= hi; n++) {
-        const int64_t sc = (chunks + n - 1) / n;
-        const size_t bytes = part_bytes(nbh, (chunks + sc - 1) / sc, R);
-        if (bytes > room && !forced) continue;
-        s.img = bytes <= room && room - bytes >= img_bytes ? img : INFINITY;
-        const pre_choice c = pre_cost(s, (uint32_t) n);
+    uint32_t last = 0;
+    for (uint32_t n = (uint32_t) lo; n <= (uint32_t) n_max; n++) {
+        const uint32_t sc = (s.chunks + n - 1) / n;
+        if (sc == last) continue;   // the same split length as a smaller count, which costs less
+        last = sc;
+        s.img = n <= n_img ? img : INFINITY;
+        const pre_choice c = pre_cost(s, n, sc);
         if (c.cost < choice->cost) { *choice = c; best = n; }
     }
     return best;
