@@ -238,7 +238,10 @@ int qwfn_qsa_select_cells(const uint16_t * pool, size_t pool_nb1, int64_t n_bloc
  * beta: F32 [T][n_v]; state: F32 [n_v][head_dim][head_dim], updated in place
  * (rs_state); out: F32 [T][n_v][head_dim]; snap: n_snap <= T-1 slots at
  * snap_stride_bytes, slot s-1 receiving the state s tokens back (the
- * rollback slots rb_rs_). head_dim = 128. Device memory throughout. */
+ * rollback slots rb_rs_). head_dim = 128. Device memory throughout. A sequence
+ * cut into calls in another way gives the same bits while every call has fewer than
+ * 12 tokens before its last n_snap + 1 (before its end without snapshots), and
+ * the same to float rounding otherwise. */
 int qwfn_gated_delta_net(const float * q, int64_t q_token_stride, const float * k, int64_t k_token_stride,
                          const float * v, int64_t v_token_stride, const float * g, const float * beta, int32_t T,
                          int32_t n_k_heads, int32_t n_v_heads, int32_t head_dim, float scale, float * state, float * out,

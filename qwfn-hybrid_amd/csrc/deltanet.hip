@@ -158,7 +158,7 @@ __global__ __launch_bounds__(DN_WAVES * 64) void k_gated_delta_net(dn_args a) {
 // ---------------------------------------------------------------- many tokens
 //
 // The same rule for chunks of 16 tokens, as matrix products on the f32 matrix
-// cores (v_mfma_f32_16x16x4_f32). With e_t = exp(g_t), D_ij = e_{j+1} .. e_i
+// cores (v_mfma_f32_16x16x4_f32): the chunkwise (WY) form of the gated delta rule. With e_t = exp(g_t), D_ij = e_{j+1} .. e_i
 // (j <= i), c_i = e_0 .. e_i within the chunk and S0 the state before it:
 //   d    = (I + A)^-1 b (v - c (K S0)),  A_ij = b_i D_ij (k_i . k_j) for j < i
 //   out  = scale (c (Q S0) + (D o QK^T) d)        (D o QK^T: j <= i only)
@@ -182,6 +182,13 @@ __global__ __launch_bounds__(DN_WAVES * 64) void k_gated_delta_net(dn_args a) {
 // recurrence; a product with the zeros of the triangular matrices would carry
 // that into earlier tokens, so the right-hand sides and the solved d of such
 // tokens enter the products as 0 and the column is set to NaN from i on.
+//
+// Rounding: with isotropic keys the error against float64 is the token form's or
+// less (T 512 5.9e-7 for 6.2e-7); with keys and queries around one direction and
+// beta near 1, c (Q S0) and (D o QK^T) d cancel and the outputs' is larger: mean
+// cosine 0.74 2.8e-7 for 0.75e-7 at T 16, 3.3e-7 for 1.7e-7 at T 256 (the state's
+// 2.1e-7 for 1.3e-7, 5.85e-7 for 5.9e-7). The matrices' sums, P and the output in
+// double bring 1.8e-7 and 2.4e-7 for 3.5% of the time; not kept.
 //
 // What bounds it: the token-by-token kernel is a chain of T steps of 0.68 us (a
 // barrier and two cross-wave sums each); here a group of 64 tokens takes 8.6 us,
