@@ -4146,6 +4146,12 @@ __global__ __launch_bounds__(VS_WAVES * 64, 2) void k_fa_vs(fa_args a) {
 // three steps ahead, the first ones under the softmax (352, 355 against 349).
 
 constexpr int PRE_WAVES = 8;
+// The reference of a row's exponentials lies this far (log2) below its maximum, so that a new maximum's P is 4;
+// with RESCALE_SLACK P stays <= 2^8 as without. P d_v goes to the matrix cores as f16 hi + lo, which cannot hold
+// less than 2^-25 of it, and the longer a split, the more keys lie that far below its maximum: against float64,
+// 24 heads, 300 queries at 9000 keys (4 splits) 6.3e-6 without, 2.0e-6 with; one split 1.3e-5 and 4.3e-6; the
+// same time. 2^4 gives 8.0e-7 and leaves the maximum less room to lag (512 x 16 at 2048 keys 67.5 -> 67.9 us).
+constexpr float PRE_LIFT = 2.f;
 constexpr int PRE_ROWS  = 16 * PRE_WAVES;                 // 128 query rows per block
 constexpr int PRE_CK    = 64;                             // keys per chunk
 constexpr int PRE_KB    = PRE_CK * SEG;                   // 17408: one tensor's rows of a chunk
@@ -4647,8 +4653,8 @@ __global__ __launch_bounds__(PRE_WAVES * 64, 2) void k_fa_pre(fa_args a) {
             const bool grow = mloc > m_run + RESCALE_SLACK;
             float alpha = 1.f;
             if (grow) {
-                alpha = __builtin_amdgcn_exp2f(m_run - mloc);
-                m_run = mloc;
+                alpha = __builtin_amdgcn_exp2f(m_run - (mloc - PRE_LIFT));
+                m_run = mloc - PRE_LIFT;
             }
             const float m_use = m_run == -INFINITY ? 0.f : m_run;
             float lsum = 0.f;
